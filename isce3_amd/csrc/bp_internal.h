@@ -136,7 +136,12 @@ struct OutDesc {
     float2* out;                // complex64 [length x width]
     float* height;              // optional float32 [length x width]
     int32_t* failed;            // per-grid flag: some pixel failed to converge
-    void* pad2_;
+    // strips of the line-interpolated split sum: strip_rows x 64 pixels, row
+    // (y, x) of strips with its StripInfo at strip_info + y strips_x + x; the
+    // batch's strips are numbered consecutively, column by column in a grid
+    int32_t strip_rows, strips_x, strips_y, pad2_;
+    int64_t strip_seq;          // first strip of this grid in the batch
+    int64_t strip_info;         // StripInfo of this grid's strip (0, 0)
 };
 
 // Counts of one (batched) call, stored on the device directly in front of its
@@ -148,8 +153,85 @@ struct BatchHeader {
     int64_t n_geom_groups;      // groups of four geometry wavefronts (lane_rows per tile)
     int32_t n_grids;
     int32_t lane_rows;
+    int64_t n_strips;           // strips of all grids
 };
-static_assert(sizeof(BatchHeader) == 32, "BatchHeader layout");
+static_assert(sizeof(BatchHeader) == 40, "BatchHeader layout");
+
+// Line-interpolated split sum (bp_lines.hip).
+constexpr int kStripLines = 64;      // lines per strip, at most
+// degree of the tap weight polynomials in the cell: 7 for even kernels, 8 for
+// odd ones, whose taps end away from a zero of the sinc (worst weight error
+// 9e-6 and 2e-6 of the peak for the widths 8 and 9; 5.5e-5 for 9 at degree 7)
+constexpr int kLineDegree = 8;
+__host__ __device__ constexpr int line_degree(int w) { return w % 2 == 0 ? 7 : 8; }
+constexpr int kLineTaps = 5;         // distinct taps of an even kernel, widths up to 9
+constexpr int kEndDegree = 4;        // weights of the taps at a cell's end
+// Limits a strip has to keep, at the ends of its lines' common pulses:
+constexpr float kLineMaxShift = 0.33f;   // bins between a line and the reference line
+constexpr double kLineMaxSlope = 1.0;    // cycles per pulse
+// phase (rad) a line gathers over half a chunk against the reference line,
+// plus pi times its bins off: what the 6 or 8 nodes interpolate (the residue
+// is x^N / (N! 2^(N-1)) at most: 1.5e-4 for x = 2.4 and N = 8, 1.2e-4 for x =
+// 1.15 and N = 6, each ten times smaller as an average over the chunk, the
+// lines and the band)
+constexpr float kLineBound8 = 2.65f, kLineBound6 = 1.35f;
+constexpr float kLineSlopeTol = 1e-4f;   // rad: a line's phase off the nodes' at a chunk's end
+// A line's position off the nodes' (bins), where pixels differ by their
+// tropospheric delay: up to kLinePosTol it is left out (1.6e-4 of a sample in
+// the middle of the band, a tenth of that over a strip's lines), up to
+// kLinePosMax the sums of the samples' derivatives at four nodes bring it in.
+// It has to be the same at both ends of the aperture to kLinePosTol.
+constexpr float kLinePosTol = 1e-4f, kLinePosMax = 3e-3f;
+constexpr int kSlopeNodes = 4;
+constexpr float kLineColumnTol = 0.06f;  // bins: fractional positions of the columns
+
+// Pulses of a strip: k0 .. k1 by some pixel, f0 .. f1 by all; chunks of
+// 2^chunk_log2 pulses (absolute multiples) from slot0.
+struct StripInfo {
+    int32_t k0, k1, f0, f1;
+    int32_t ok;
+    int32_t slot0, nslots;
+    int32_t slopes;          // the lines' positions need the samples' derivatives
+};
+
+// Per-pixel record of the line-interpolated sum (in the place of PixSplit):
+// the phase in cycles p0 + a1 j + .. + a4 j^4, j = k - k0, and the range bin
+// ub + uf + (phase - p0) / (fc dtau).
+struct alignas(16) PixLine {
+    double p0, a1, a2, a3, a4;
+    float uf;
+    int32_t ub;
+    int32_t kstart, kstop;
+    float du;                // bins off the position the nodes interpolate
+    int32_t pad_;
+};
+static_assert(sizeof(PixLine) == 64, "PixLine layout");
+
+struct LineArgs {
+    const BatchHeader* batch;
+    PixLine* rec;
+    StripInfo* info;
+    int32_t* n_bad;                      // strips left to the pixel-by-pixel sum
+    const float2* rc;                    // range-compressed pulses [na x nr]
+    int64_t nr;
+    double inv_k;                        // 1 / (fc dtau): cycles -> range bins
+    double in_r0, inv_dr;                // input grid: starting range, 1 / spacing
+    int64_t s_begin, s_end;              // strips of this launch
+    // Pulses in device memory a part at a time: the chunks that begin in
+    // [q_begin, q_end), multiples of 64, with the running FP64 sums of
+    // strip_lines kept in `carry` between the parts (null: all at once).
+    int32_t q_begin, q_end, q_first, pad_;
+    double2* carry;                      // [strip][segment][64 lines][64]
+    int32_t slots;                       // chunks per strip in the workspace
+    int32_t chunk_log2;
+    int32_t n_sums, tropo;               // sums per chunk: 8 nodes, and with a
+                                         // tropospheric delay kSlopeNodes slopes
+    float2* sums;                        // [strip][slot][n_sums][64]
+    float2* parts;                       // [strip][segment][64 lines][64]
+    unsigned long long* cross;           // [strip][slot][8 nodes]
+    float farrow[kLineDegree + 1][kLineTaps];
+    float w_in[kEndDegree + 1], w_out[kEndDegree + 1];
+};
 
 __host__ __device__ inline const OutDesc* batch_grids(const BatchHeader* b)
 {
@@ -173,8 +255,10 @@ struct GeomArgs {
     G2RParams g2r;
     PixGeom* geom;              // plain records (always written)
     PixSplit* split;            // split records (when want_split)
-    int32_t* flags;             // [0] any failed, [1] out of range
+    int32_t* flags;             // [0] any failed, [1] out of range, [2] strips
+                                // left to the pixel-by-pixel split sum
     unsigned long long* updates;
+    const StripInfo* strips;    // line-interpolated sum's strips, or null
 };
 
 struct SumArgs {
@@ -199,6 +283,8 @@ struct SumArgs {
     double inv_dtau;            // 1 / dtau
     const double2* tab2;        // plain: (t_i, t_{i+1} - t_i) per table entry, as doubles
     double fold_c[4];           // split: n, C(n,2), C(n,3), C(n,4) for n = chunk
+    const StripInfo* strips;    // split: strips summed by line interpolation, or null
+    const int32_t* n_bad;       // strips that are not
 };
 
 // Host launchers (defined in bp_kernels.hip).  `grid` is the number of
@@ -214,6 +300,16 @@ hipError_t launch_sum_plain(const SumArgs& args, int width, int grid, hipStream_
 hipError_t launch_sum_split(const SumArgs& args, int width, int grid, bool staged, bool pair,
                             hipStream_t stream);
 int sum_blocks_per_cu(int precision, int width, bool staged, bool pair);
+// Line-interpolated split sum (bp_lines.hip): workspace bytes per strip and
+// its placement, kernels and their grids.
+enum LineKernel : int { kLineFit = 0, kLineNodes, kLineLines, kLineEnds, kLineSum };
+size_t line_strip_bytes(int slots, int n_sums);
+size_t line_carry_bytes();
+void line_place(LineArgs& a, unsigned char* ws, int64_t n_strips);
+const void* line_kernel_fn(int which, int width);
+int64_t line_grid(int which, int slots, int64_t n_strips);
+hipError_t launch_strip_fit(const GeomArgs& g, const LineArgs& a, int64_t grid, hipStream_t stream);
+hipError_t launch_strips(const LineArgs& a, int width, bool last, hipStream_t stream);
 // [kmin, kmax) of each band of band_rows output lines (n_bands workgroups).
 hipError_t launch_band_window(const PixGeom* geom, int64_t length, int64_t width, int band_rows,
                               int64_t n_bands, int32_t* win, hipStream_t stream);

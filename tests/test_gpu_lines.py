@@ -1,0 +1,125 @@
+"""The line-interpolated split sum (strips of output lines focused from a few
+of them) against the all-FP64 oracle, on random pulses and a full synthetic
+aperture (about 4,000 pulses): strip heights and widths at their edges, both
+kernel widths it takes, straight and curved orbits over rough terrain, and
+blocks where it takes none or only some of the strips.
+
+Tolerances, from the method's own bounds: the tap weights are within 1e-5 of
+the tabulated kernel at any position (2e-6 at width 9), which white pulses turn
+into at most sqrt(8) x 1e-5 = 2.8e-5 relative; the node interpolation leaves at
+most 1.5e-4 at a chunk's end, a tenth of that on average; FP32 phases of 16
+cycles 6e-6 rad: 6e-5 together.  Over rough terrain from a curved orbit a strip
+may stray 1e-4 rad from its nodes at a chunk's ends, 6e-5 RMS over the chunk:
+1e-4 with the other terms.  The pixel-by-pixel sum's weight table is good to
+1.5e-4 on white pulses: 2e-4 where it takes part."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import complex_rel_error
+
+pytestmark = pytest.mark.gpu
+
+NA, NR = 4600, 192
+
+
+def _scene(width=8, orbit="straight", relief=0.0, doppler=0.0):
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import KnabKernel, LUT2d, Orbit, TabulatedKernelF32
+    from isce3_amd.geometry import DEMInterpolator
+    if orbit == "straight":
+        orb = sim.straight_orbit()
+    else:
+        t = -50.0 + 10.0 * np.arange(11)
+        r = sim.WGS84_A + sim.ALTITUDE
+        a = sim.SPEED / r * t
+        orb = Orbit.from_arrays(
+            sim.EPOCH, -50.0, 10.0,
+            np.stack([r * np.cos(a), 0 * a, r * np.sin(a)], axis=1),
+            sim.SPEED * np.stack([-np.sin(a), 0 * a, np.cos(a)], axis=1))
+    in_grid = sim._grid(-0.5 * NA / sim.PRF, sim.PRF, sim.R0, sim.DR, NA, NR)
+    dem = DEMInterpolator(50.0)
+    if relief:
+        dem = sim._dem_around(orb, in_grid, 256, 30.0, 0.8, relief, 3)
+    xs = sim.R0 + sim.DR * np.array([-20.0, NR + 20.0])
+    ys = np.array([-45.0, 45.0])
+    lut = LUT2d(xs, ys, np.full((2, 2), doppler)) if doppler else LUT2d()
+    rng = np.random.default_rng(5)
+    raw = (rng.standard_normal((NA, NR)) + 1j * rng.standard_normal((NA, NR))).astype(np.complex64)
+    kernel = TabulatedKernelF32(KnabKernel(float(width), 0.8), 2048)
+    return orb, RadarGeometry(in_grid, orb, lut), dem, raw, kernel
+
+
+def _run(scene, rows, cols, c0=40, dr=None, prf=None, tropo="nodelay", options=None):
+    """(GPU split result, FP64 oracle) of a block of rows x cols pixels."""
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import LUT2d
+    from isce3_amd.focus import backproject
+    orb, in_geom, dem, raw, kernel = scene
+    prf = prf or sim.PRF
+    grid = sim._grid(-0.5 * rows / prf + 0.3 / prf, prf, sim.R0 + (c0 + 0.37) * sim.DR,
+                     dr or sim.DR, rows, cols)
+    og = RadarGeometry(grid, orb, LUT2d())
+    out = np.empty(grid.shape, np.complex64)
+    err = backproject(out, og, raw, in_geom, dem, sim.FC, 6.0, kernel, tropo, precision="split",
+                      options=options)
+    ref, _, _, rc = oracle.backproject(og, raw, in_geom, dem, sim.FC, 6.0, kernel, tropo, mode=1,
+                                       kernel_bandwidth=0.8)
+    assert err == (rc == 6)
+    rel = complex_rel_error(out, ref)
+    print(f"[lines] {rows}x{cols} rel={rel:.2e}", flush=True)
+    assert (np.isnan(out) == np.isnan(ref)).all()
+    return rel
+
+
+@pytest.mark.parametrize("width", [8, 9])
+@pytest.mark.parametrize("rows,cols", [(1, 64), (5, 3), (16, 65), (33, 64), (64, 20), (65, 63),
+                                       (130, 40)])
+def test_strip_edges_match_fp64_oracle(torch_gpu, width, rows, cols):
+    assert _run(_scene(width), rows, cols) <= 6e-5
+
+
+@pytest.mark.parametrize("orbit,relief,tropo", [("straight", 100.0, "tsx"),
+                                                ("circular", 0.0, "nodelay"),
+                                                ("circular", 100.0, "tsx")])
+def test_orbits_and_terrain_match_fp64_oracle(torch_gpu, orbit, relief, tropo):
+    assert _run(_scene(8, orbit, relief), 96, 70, tropo=tropo) <= 1e-4
+
+
+@pytest.mark.parametrize("kw", [dict(dr=9.0), dict(prf=400.0), dict(c0=-30), dict(c0=150)])
+def test_strips_left_to_the_pixel_sum(torch_gpu, kw):
+    """Output range spacing off the input's, lines too far apart, and blocks
+    whose first or last columns' taps leave the range line (a strip of 64
+    columns beside one that qualifies)."""
+    assert _run(_scene(8), 40, 100 if "c0" in kw else 40, **kw) <= 2e-4
+
+
+def test_native_doppler(torch_gpu):
+    """A squinted aperture: ranges of adjacent lines are too far apart at its
+    far end, so the strips take the pixel-by-pixel sum."""
+    assert _run(_scene(8, doppler=400.0), 48, 64) <= 2e-4
+
+
+def test_whole_and_band_by_band_agree(torch_gpu):
+    """Pulses in host memory under a budget below a strip's window: the strip's
+    pulses go through the device in parts, with the same result to the bit."""
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import LUT2d
+    from isce3_amd.focus import backproject
+    orb, in_geom, dem, raw, kernel = _scene(9)
+    grid = sim._grid(-0.5 * 150 / sim.PRF, sim.PRF, sim.R0 + 40 * sim.DR, sim.DR, 150, 70)
+    og = RadarGeometry(grid, orb, LUT2d())
+    outs = []
+    for budget in (0, 4300 * NR * 8, 4110 * NR * 8):
+        out = np.empty(grid.shape, np.complex64)
+        st = {}
+        backproject(out, og, raw, in_geom, dem, sim.FC, 6.0, kernel, "nodelay",
+                    precision="split", max_window_bytes=budget, stats=st)
+        print(f"[lines] budget {budget}: {st['bands']} bands, {st['window_pulses']} pulses",
+              flush=True)
+        outs.append(out)
+    np.testing.assert_array_equal(outs[1], outs[0])
+    np.testing.assert_array_equal(outs[2], outs[0])
