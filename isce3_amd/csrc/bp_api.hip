@@ -1123,7 +1123,6 @@ void build_step(Step& sp, const StaticData& st, const Scratch& sc, const CallArg
     std::memset(&sa, 0, sizeof(sa));
     sa.batch = batch;
     sa.nr = gi.width;
-    sa.na = (int32_t)gi.length;
     sa.swst = swst;
     sa.dtau = dtau;
     sa.fc = a.fc;

@@ -279,7 +279,6 @@ struct SumArgs {
     const float* poly;          // polyphase weights (split): (rows+1) x poly_row_floats(W)
     const float* poly2;         // two-line weights (split, lane_rows 2): pair_table_floats(W)
     float zscale2;              // -2^pair_q_log2(W) * inv_k
-    int32_t na;                 // pulses
     int32_t exact_width;        // plain: 2 * halfwidth == W (no tap lies past the half width)
     double inv_dtau;            // 1 / dtau
     const double2* tab2;        // plain: (t_i, t_{i+1} - t_i) per table entry, as doubles

@@ -379,8 +379,6 @@ __device__ inline void for_each_tile(const BatchHeader* batch, Body&& body)
 // kExact: 2 * halfwidth == W, so no tap lies past the half width.
 // `tab2` is the table in LDS or in global memory: each caller passes one of
 // the two, so that the reads compile to LDS or global loads.
-constexpr int kPlainChunk = 64;
-
 template<int W, bool kExact>
 __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const OutDesc& od,
                                   int64_t tile, int lane)
@@ -403,18 +401,16 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
     const double an_max = a.halfwidth * rdx;
     const int ntab = a.ntab;
 
-    const auto* pulses = uniform_ptr(a.pulse_pv);
-    // delay at pulse k (wave-uniform: its record comes through the scalar cache)
-    auto delay = [&](int k) {
-        const auto* pv = pulses + kPulseRecDoubles * (int64_t)k;
+    double acc_re = 0., acc_im = 0.;
+    for (int k = kw0; k < kw1; ++k) {
+        if (k < ks || k >= ke) continue;
+        // the pulse record (k is wave-uniform) through the scalar cache
+        const auto* pv = uniform_ptr(a.pulse_pv) + kPulseRecDoubles * (int64_t)k;
         const V3 r{x.x - pv[0], x.y - pv[1], x.z - pv[2]};
         const double rv = r.x * pv[3] + r.y * pv[4] + r.z * pv[5];
         const double rn = sqrt_normal(r.x * r.x + r.y * r.y + r.z * r.z);
-        return tau_atm + (rv - kC * rn) * pv[6];
-    };
-    double acc_re = 0., acc_im = 0.;
-    // adds pulse k's sample at range bin u times the phasor cs + i sn
-    auto add = [&](int k, double u, double cs, double sn) {
+        const double tau = tau_atm + (rv - kC * rn) * pv[6];
+        const double u = (tau - a.swst) * a.inv_dtau;
         const double low = ((W % 2 == 0) ? ceil(u) : round(u)) - (double)(W / 2);
         const double a0 = (low - u) * rdx;
         float w[W];
@@ -447,65 +443,13 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
                 sim = fmaf(w[m], d.y, sim);
             }
         }
+        double sn, cs;
+        sincos_turns(a.fc * tau, &sn, &cs);
         const double dre = (double)sre, dim = (double)sim;
         acc_re = fma(dre, cs, acc_re);
         acc_re = fma(-dim, sn, acc_re);
         acc_im = fma(dre, sn, acc_im);
         acc_im = fma(dim, cs, acc_im);
-    };
-    // Pulses in chunks of kPlainChunk: the delay is a cubic of the pulse
-    // index through its values at four of the chunk's pulses (the fourth
-    // difference leaves 1.3e-10 cycles at 850 km, 7.5 km/s and 1520 Hz over 64
-    // pulses, less than the rounding of fc tau, 9e-10); the range bin steps by
-    // its forward differences and the phasor by the products of its
-    // differences' phasors, three adds and ten FMAs per pulse where the delay
-    // (a square root) and the sine and cosine of its phase took 58
-    // instructions.
-    // The chunks begin at multiples of kPlainChunk, so that a pixel's values do
-    // not depend on the pixels that share its wavefront; a last chunk cut off
-    // by the data's end is summed pulse by pulse.
-    const int na64 = a.na / kPlainChunk * kPlainChunk;
-    const double e1 = 19., e2 = 44., e3 = 61., e0 = 2.;   // Chebyshev points of 64 pulses
-    for (int k = kw0 / kPlainChunk * kPlainChunk; k < min(kw1, na64); k += kPlainChunk) {
-        const double t0 = delay(k + 2), t1 = delay(k + 19), t2 = delay(k + 44), t3 = delay(k + 61);
-        const double f01 = (t1 - t0) * (1. / (e1 - e0)), f12 = (t2 - t1) * (1. / (e2 - e1)),
-                     f23 = (t3 - t2) * (1. / (e3 - e2));
-        const double f012 = (f12 - f01) * (1. / (e2 - e0)), f123 = (f23 - f12) * (1. / (e3 - e1));
-        const double c3 = (f123 - f012) * (1. / (e3 - e0));
-        // coefficients of (pulse - k)^i, then forward differences
-        const double c2 = fma(-(e0 + e1 + e2), c3, f012);
-        const double c1 = fma(e0 * e1 + e0 * e2 + e1 * e2, c3, fma(-(e0 + e1), f012, f01));
-        const double tau0 = fma(-e0 * e1 * e2, c3, fma(e0 * e1, f012, fma(-e0, f01, t0)));
-        const double g1 = c1 + c2 + c3, g2 = fma(6., c3, 2. * c2), g3 = 6. * c3;
-        double u = (tau0 - a.swst) * a.inv_dtau;
-        double u1 = g1 * a.inv_dtau, u2 = g2 * a.inv_dtau;
-        const double u3 = g3 * a.inv_dtau;
-        double zr, zi, wr, wi, vr, vi;
-        sincos_turns(a.fc * tau0, &zi, &zr);
-        sincos_turns(a.fc * g1, &wi, &wr);
-        sincos_turns(a.fc * g2, &vi, &vr);
-        const double eps = 2. * kPi * a.fc * g3;   // ~3e-10 rad: 1 + i eps
-        for (int j = 0; j < kPlainChunk; ++j) {
-            if (k + j >= ks && k + j < ke) add(k + j, u, zr, zi);
-            u += u1;
-            u1 += u2;
-            u2 += u3;
-            const double zt = fma(zr, wr, -zi * wi), wt = fma(wr, vr, -wi * vi);
-            zi = fma(zr, wi, zi * wr);
-            zr = zt;
-            wi = fma(wr, vi, wi * vr);
-            wr = wt;
-            const double vt = fma(-eps, vi, vr);
-            vi = fma(eps, vr, vi);
-            vr = vt;
-        }
-    }
-    for (int k = max(kw0, na64); k < kw1; ++k) {
-        if (k < ks || k >= ke) continue;
-        const double tau = delay(k);
-        double sn, cs;
-        sincos_turns(a.fc * tau, &sn, &cs);
-        add(k, (tau - a.swst) * a.inv_dtau, cs, sn);
     }
     if (valid) {
         const float nanf_ = __builtin_nanf("");
@@ -520,8 +464,7 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
 constexpr int kMaxTab2Lds = 4096;
 
 template<int W>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-void sum_plain_kernel(SumArgs a)
+__global__ __launch_bounds__(256) void sum_plain_kernel(SumArgs a)
 {
     const int64_t ng = uniform64(a.batch->n_groups);
     if ((int64_t)blockIdx.x >= ng) return;
