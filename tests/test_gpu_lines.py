@@ -113,7 +113,10 @@ def test_whole_and_band_by_band_agree(torch_gpu):
     grid = sim._grid(-0.5 * 150 / sim.PRF, sim.PRF, sim.R0 + 40 * sim.DR, sim.DR, 150, 70)
     og = RadarGeometry(grid, orb, LUT2d())
     outs = []
-    for budget in (0, 4300 * NR * 8, 4110 * NR * 8):
+    # whole; bands of one strip row each (64 lines' window); parts of a strip's window
+    windows = [0]
+    for windows_of in (0, 1, 2):
+        budget = windows[windows_of] * NR * 8
         out = np.empty(grid.shape, np.complex64)
         st = {}
         backproject(out, og, raw, in_geom, dem, sim.FC, 6.0, kernel, "nodelay",
@@ -121,5 +124,10 @@ def test_whole_and_band_by_band_agree(torch_gpu):
         print(f"[lines] budget {budget}: {st['bands']} bands, {st['window_pulses']} pulses",
               flush=True)
         outs.append(out)
+        if not windows_of:
+            strip = st["window_pulses"] - 150 + 64
+            windows += [strip + 20, strip - 40]
+        else:
+            assert st["bands"] >= 2
     np.testing.assert_array_equal(outs[1], outs[0])
     np.testing.assert_array_equal(outs[2], outs[0])
