@@ -120,9 +120,20 @@ __host__ __device__ constexpr int pair_table_floats(int w)
 }
 
 // Doubles per pulse of the plain sum's per-pulse record: platform position
-// (3), velocity (3), 2 / (|v|^2 - c^2) (the bistatic delay's factor) and one
-// of padding.
+// (3), velocity (3), 2 / (|v|^2 - c^2) (the bistatic delay's factor) and the
+// position's difference from the cubic of its chunk.
 constexpr int kPulseRecDoubles = 8;
+
+// The plain sum takes pulses in chunks of kPlainChunk (absolute multiples) and
+// interpolates a pixel's delay between four of them (near the Chebyshev points
+// of the chunk).
+constexpr int kPlainChunk = 64;
+constexpr int kPlainNode[4] = {2, 19, 44, 61};
+// A pulse's position less the cubic through the nodes' positions, kPosQ
+// steps per metre in three 21-bit fields, or kPosNone in a chunk where some do
+// not fit (2.4e-7 m) or that the data's end cuts off: delays are evaluated there.
+constexpr double kPosQ = 4398046511104.0;  // 2^42
+constexpr unsigned long long kPosNone = 1ull << 63;
 
 // One output grid of a (batched) call.  Wavefront tiles of all grids are
 // numbered consecutively: grid g owns [seq_base, seq_base + map.n_tiles).

@@ -1,0 +1,62 @@
+"""The plain sum's chunks of 64 pulses (delay by a cubic, phasor by recurrence)
+against the oracle: raw sets shorter than a chunk, at its multiples and
+off them, windows that begin and end inside chunks, and low short-range
+tracks where the cubic fits all, none or some of the pixels.
+
+Tolerance: weights and products in FP32, up to 9 taps of 6e-8 each in weight, product
+and sum, add as random errors to at most 3e-7 of a pixel; a cubic within 1e-9
+cycles (6e-9 rad) or a few ulp of the phase (1e-8 rad) and a phasor within 2e-8
+are below that: 5e-7."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import complex_rel_error
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(na, ds, rows=21, cols=35, altitude=None, speed=None, prf=None, r0=None, width=8):
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import KnabKernel, LUT2d, Orbit, TabulatedKernelF32
+    from isce3_amd.focus import backproject
+    from isce3_amd.geometry import DEMInterpolator
+    prf, r0, nr = prf or sim.PRF, r0 or sim.R0, 96
+    orb = sim.straight_orbit()
+    if altitude:
+        t = -50.0 + 10.0 * np.arange(11)
+        pos = np.stack([0 * t + sim.WGS84_A + altitude, 0 * t, speed * t], axis=1)
+        orb = Orbit.from_arrays(sim.EPOCH, -50.0, 10.0, pos,
+                                np.repeat([[0.0, 0.0, speed]], len(t), axis=0))
+    in_grid = sim._grid(-0.5 * na / prf, prf, r0, sim.DR, na, nr)
+    in_geom = RadarGeometry(in_grid, orb, LUT2d())
+    grid = sim._grid(-0.5 * rows / prf, prf, r0 + 12.3 * sim.DR, sim.DR, rows, cols)
+    og = RadarGeometry(grid, orb, LUT2d())
+    rng = np.random.default_rng(na)
+    raw = (rng.standard_normal((na, nr)) + 1j * rng.standard_normal((na, nr))).astype(np.complex64)
+    kernel = TabulatedKernelF32(KnabKernel(float(width), 0.8), 2048)
+    dem = DEMInterpolator(50.0)
+    out = np.empty(grid.shape, np.complex64)
+    backproject(out, og, raw, in_geom, dem, sim.FC, ds, kernel, "nodelay", precision="plain")
+    ref, _, _, _ = oracle.backproject(og, raw, in_geom, dem, sim.FC, ds, kernel, "nodelay", mode=0)
+    assert (np.isnan(out) == np.isnan(ref)).all()
+    rel = complex_rel_error(out, ref)
+    print(f"[plain chunks] na={na} ds={ds} rel={rel:.2e}", flush=True)
+    assert rel <= 5e-7
+
+
+@pytest.mark.parametrize("width", [8, 9])
+@pytest.mark.parametrize("na", [1, 63, 64, 65, 200, 256])
+def test_every_pulse(torch_gpu, na, width):
+    _check(na, 6.0, width=width)
+
+
+@pytest.mark.parametrize("na", [300, 321])
+def test_windows_inside_chunks(torch_gpu, na):
+    _check(na, 200.0)
+
+
+@pytest.mark.parametrize("prf", [100.0, 700.0, 3000.0])
+def test_short_ranges(torch_gpu, prf):
+    _check(330, 6.0, altitude=3000.0, speed=120.0, prf=prf, r0=5000.0)
