@@ -112,6 +112,7 @@ struct StaticData {
 struct Scratch {
     DevBuf geom, split, flags, desc;
     DevBuf strips, lines;   // line-interpolated sum: StripInfo, workspace
+    DevBuf parts;           // plain sum: segment sums of small batches
 };
 
 // Buffers of the host-input path (bp_backproject_host): device pulse windows,
@@ -679,7 +680,7 @@ void free_static(StaticData& s)
 
 void free_scratch(Scratch& s)
 {
-    DevBuf* bufs[] = {&s.geom, &s.split, &s.flags, &s.desc, &s.strips, &s.lines};
+    DevBuf* bufs[] = {&s.geom, &s.split, &s.flags, &s.desc, &s.strips, &s.lines, &s.parts};
     for (DevBuf* b : bufs)
         if (b->ptr && !b->fixed) (void)hipFree(b->ptr);
 }
@@ -991,6 +992,7 @@ struct Step {
     int flag_words;
     hipEvent_t ev[3];  // null: no timing
     // line-interpolated sum (split; lines false: every pixel at every pulse)
+    int segs;              // plain: segments with wavefronts of their own
     bool lines;
     bp::LineArgs la;
     int64_t n_strips;      // of the batch (the fit's grid)
@@ -1051,6 +1053,25 @@ LinePlan plan_lines(const CallArgs& a, int width, const Opts& o)
     p.strip_bytes = bp::line_strip_bytes(p.slots, p.table.n_sums);
     p.on = p.strip_bytes <= kLineBytes;
     return p;
+}
+
+// Segments of the plain sum that get wavefronts of their own (0: none).  The
+// chip holds 4,096 of its wavefronts: 256 x 256 pixels are 1,024, each with
+// 512 pulses to sum one after the other, and 301 x 1003 pixels are 4,718, so that
+// a second round runs 15% full.  By segments these take 0.34 instead of
+// 0.50 ms and 5.8 instead of 8.3 ms.  From four rounds on (kPlainWaves) the
+// last one costs less than the segments' sums, which are kept while they fit
+// kPartBytes.
+constexpr int64_t kPlainWaves = 16384;
+constexpr size_t kPartBytes = size_t(256) << 20;
+
+int plain_segments(const CallArgs& a, int64_t n_seq, int64_t n_rec)
+{
+    if (a.precision != BP_PRECISION_PLAIN || n_seq >= kPlainWaves) return 0;
+    const int64_t segs = (a.in_geometry->grid.length + bp::kPlainSeg - 1) / bp::kPlainSeg;
+    if (segs < 2 || segs > 65535 || (double)segs * n_rec * sizeof(double2) > (double)kPartBytes)
+        return 0;
+    return (int)segs;
 }
 
 // Strips whose workspace a call with n of them takes at once.
@@ -1164,6 +1185,7 @@ void build_step(Step& sp, const StaticData& st, const Scratch& sc, const CallArg
     sp.flag_words = 0;
     sp.ev[0] = sp.ev[1] = sp.ev[2] = nullptr;
     sp.lines = false;
+    sp.segs = 0;
 }
 
 void set_lines(Step& sp, const LinePlan& p, const Scratch& sc, const CallArgs& a, int64_t n,
@@ -1218,7 +1240,7 @@ int enqueue_sum(const Step& sp, const bp::BatchHeader* batch, const float2* rc, 
         }
     }
     if (sp.precision == BP_PRECISION_PLAIN)
-        BP_HIP_CHECK(bp::launch_sum_plain(sa, sp.width, plain_grid, s));
+        BP_HIP_CHECK(bp::launch_sum_plain(sa, sp.width, plain_grid, sp.segs, s));
     else
         BP_HIP_CHECK(bp::launch_sum_split(sa, sp.width, sp.sum_grid, sp.staged, sp.pair, s));
     return BP_SUCCESS;
@@ -1278,6 +1300,7 @@ struct Carve;
 int carve_call(Carve& cv, const CallArgs& a, int width, int n_blocks, int64_t npix,
                StaticData& st, Scratch& sc);
 int64_t carve_lines(Carve& cv, const LinePlan& p, int64_t n_strips, Scratch& sc);
+int carve_parts(Carve& cv, size_t bytes, Scratch& sc);
 
 int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blocks,
                const bp_options* options, void* stream, int* any_failed, bp_stats* stats,
@@ -1318,6 +1341,13 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
         return rc;
     const int64_t n_rec = npix;
 
+    int segs = plain_segments(a, hdr.n_seq, n_rec);
+    if (segs > 0) {
+        const size_t bytes = sizeof(double2) * (size_t)segs * n_rec;
+        if (carve ? carve_parts(*carve, bytes, sc) : ensure(sc.parts, bytes)) segs = 0;
+        hdr.plain_segs = segs;
+        std::memcpy(c->desc_host.data(), &hdr, sizeof(hdr));
+    }
     if ((rc = upload_static(st, a, width, s))) return rc;
     if ((rc = upload(sc.desc, c->desc_host.data(), c->desc_host.size(), s))) return rc;
     if ((rc = ensure(sc.geom, sizeof(bp::PixGeom) * n_rec))) return rc;
@@ -1339,6 +1369,11 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
     Step sp;
     build_step(sp, st, sc, a, width, o, c->n_cu);
     if (group > 0) set_lines(sp, lp, sc, a, hdr.n_strips, group);
+    if (segs > 0) {
+        sp.segs = segs;
+        sp.sa.parts = static_cast<double2*>(sc.parts.ptr);
+        sp.sa.parts_stride = n_rec;
+    }
     sp.geom_grid = (int)hdr.n_geom_groups;
     sp.fit_grid = (int)hdr.n_groups;
     sp.flag_words = 0;  // cleared above, before the pulse states
@@ -1424,6 +1459,13 @@ int carve_call(Carve& cv, const CallArgs& a, int width, int n_blocks, int64_t np
         if (cv.take(*w.b, (size_t)w.bytes) != BP_SUCCESS)
             return fail(BP_ERR_LENGTH, "bp_backproject_noalloc: scratch layout overflow");
     return BP_SUCCESS;
+}
+
+// Segment sums of the plain sum in what a no-alloc call's buffers leave.
+int carve_parts(Carve& cv, size_t bytes, Scratch& sc)
+{
+    if (cv.used > cv.cap || bytes + 256 > cv.cap - cv.used) return BP_ERR_LENGTH;
+    return cv.take(sc.parts, bytes);
 }
 
 // Workspace of the line-interpolated sum in what a no-alloc call's buffers
@@ -1911,11 +1953,13 @@ struct bp_scene {
     LinePlan lines{};          // line-interpolated sum (lane_rows 2)
     int64_t line_strips = 0;   // strips the scene holds records for, ...
     int64_t line_group = 0;    // ... and workspace for at a time
+    int64_t part_records = 0;  // plain: pixels whose segment sums the scene holds
     // A kernel node whose grid follows the batch, with its captured launch
     // parameters: the geometry pass (geometry groups), fit and plain sum (tile
-    // groups), strip fit (strips), and the kernels of the line-interpolated
+    // groups; the plain sum by segments), strip fit (strips), and the kernels of
+    // the line-interpolated
     // sum (the strips of their group, from first on, at most count).
-    enum Kind { kGeom, kTiles, kStrips };   // kStrips + a LineKernel for the others
+    enum Kind { kGeom, kTiles, kPlain, kStrips };   // kStrips + a LineKernel for the others
     struct GridNode {
         hipGraphNode_t node;
         hipKernelNodeParams params;
@@ -1975,6 +2019,10 @@ int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
     build_step(sp, sc->st, sc->sc, sc->args, sc->width, o, c->n_cu);
     if (sc->lines.on && o.lane_rows == 2 && !o.staged)
         set_lines(sp, sc->lines, sc->sc, sc->args, sc->line_strips, sc->line_group);
+    if (sc->part_records > 0) {
+        sp.sa.parts = static_cast<double2*>(sc->sc.parts.ptr);
+        sp.sa.parts_stride = sc->part_records;
+    }
     // the geometry, fit and plain-sum grids are set per replay to the batch's
     // group counts (bp_scene_focus); one workgroup at capture
     const int cap_grid = 1;
@@ -2016,9 +2064,10 @@ int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
     const bool pair = o.lane_rows == 2;
     const void* geo_fn = bp::kernel_fn(bp::dem_generic(host_dem(sc->dem)) ? 4 : 0, sc->width,
                                        o.staged, pair);
-    const void* tile_fn = sc->args.precision == BP_PRECISION_PLAIN
-                              ? bp::kernel_fn(1, sc->width, o.staged, pair)
-                              : bp::kernel_fn(3, sc->width, o.staged, pair);
+    const bool plain = sc->args.precision == BP_PRECISION_PLAIN;
+    const void* tile_fn = bp::kernel_fn(plain ? 1 : 3, sc->width, o.staged, pair);
+    const void* total_fn = plain && sc->part_records > 0 ? bp::kernel_fn(5, sc->width, false, false)
+                                                         : nullptr;
     for (hipGraphNode_t nd : nodes) {
         hipGraphNodeType type;
         if (hipGraphNodeGetType(nd, &type) != hipSuccess || type != hipGraphNodeTypeKernel) continue;
@@ -2028,6 +2077,9 @@ int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
         if (p.func == geo_fn) {
             out->nodes.push_back(gn);
         } else if (p.func == tile_fn) {
+            gn.kind = plain ? bp_scene::kPlain : bp_scene::kTiles;
+            out->nodes.push_back(gn);
+        } else if (total_fn != nullptr && p.func == total_fn) {
             gn.kind = bp_scene::kTiles;
             out->nodes.push_back(gn);
         } else if (sp.lines) {
@@ -2045,7 +2097,7 @@ int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
     }
     const size_t groups =
         sp.lines ? (size_t)((sp.n_strips + sp.group_strips - 1) / sp.group_strips) : 0;
-    const size_t want = 2 + (sp.lines ? 1 + 4 * groups : 0);
+    const size_t want = 2 + (total_fn ? 1 : 0) + (sp.lines ? 1 + 4 * groups : 0);
     if (out->nodes.size() != want) {
         (void)hipGraphDestroy(g);
         return fail(BP_ERR_HIP, "captured step is missing its kernel nodes");
@@ -2127,6 +2179,13 @@ try {
     if (hipMemsetAsync(sc->sc.flags.ptr, 0, flag_bytes, s) != hipSuccess)
         return bail(fail(BP_ERR_HIP, "hipMemsetAsync failed"));
     if ((rc = pulse_states(sc->st, sc->args, static_cast<int32_t*>(sc->sc.flags.ptr), s))) return bail(rc);
+    if (precision == BP_PRECISION_PLAIN && in_geometry->grid.length > bp::kPlainSeg) {
+        const int64_t segs = (in_geometry->grid.length + bp::kPlainSeg - 1) / bp::kPlainSeg;
+        const int64_t most = (int64_t)(kPartBytes / (segs * sizeof(double2)));
+        const int64_t n = std::min(max_pixels, std::min(most, kPlainWaves * 64));
+        if (n > 0 && ensure(sc->sc.parts, sizeof(double2) * segs * n) == BP_SUCCESS)
+            sc->part_records = n;
+    }
     {
         Opts two{};
         two.lane_rows = 2;
@@ -2216,17 +2275,22 @@ try {
     if ((rc = plan_batch(blocks, n_blocks, o, static_cast<int32_t*>(sc->sc.flags.ptr) + kFlagWords,
                          sc->h_desc, sc->max_blocks, &hdr, sc->block_of_grid)) != BP_SUCCESS)
         return rc;
+    if (sc->part_records > 0 && npix <= sc->part_records) {
+        hdr.plain_segs = plain_segments(sc->args, hdr.n_seq, npix);
+        std::memcpy(sc->h_desc, &hdr, sizeof(hdr));
+    }
     for (const bp_scene::GridNode& gn : g->nodes) {
         const int64_t n = std::min(std::max<int64_t>(hdr.n_strips - gn.first, 0), gn.count);
         int64_t grid;
         switch (gn.kind) {
         case bp_scene::kGeom: grid = hdr.n_geom_groups; break;
-        case bp_scene::kTiles: grid = hdr.n_groups; break;
+        case bp_scene::kTiles: case bp_scene::kPlain: grid = hdr.n_groups; break;
         case bp_scene::kStrips: grid = hdr.n_strips; break;
         default: grid = bp::line_grid(gn.kind - bp_scene::kStrips, sc->lines.slots, n); break;
         }
         hipKernelNodeParams p = gn.params;
-        p.gridDim = dim3((unsigned)std::max<int64_t>(grid, 1));
+        p.gridDim = dim3((unsigned)std::max<int64_t>(grid, 1),
+                         gn.kind == bp_scene::kPlain ? (unsigned)std::max(hdr.plain_segs, 1) : 1u);
         BP_HIP_CHECK(hipGraphExecKernelNodeSetParams(g->exec, gn.node, &p));
     }
     if (stats) BP_HIP_CHECK(hipEventRecord(sc->ev[0], s));

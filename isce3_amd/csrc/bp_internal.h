@@ -165,8 +165,16 @@ struct BatchHeader {
     int32_t n_grids;
     int32_t lane_rows;
     int64_t n_strips;           // strips of all grids
+    int32_t plain_segs;         // plain sum: segments summed by their own
+                                // wavefronts, 0: each wavefront takes them all
+    int32_t pad_;
 };
-static_assert(sizeof(BatchHeader) == 40, "BatchHeader layout");
+static_assert(sizeof(BatchHeader) == 48, "BatchHeader layout");
+
+// Pulses per segment of the plain sum: 512 pulses still give four wavefronts a
+// tile, and the table's copy to LDS is 1% of a segment's work.
+constexpr int kPlainSeg = 128;
+static_assert(kPlainSeg % kPlainChunk == 0, "segments of whole chunks");
 
 // Line-interpolated split sum (bp_lines.hip).
 constexpr int kStripLines = 64;      // lines per strip, at most
@@ -296,6 +304,8 @@ struct SumArgs {
     double fold_c[4];           // split: n, C(n,2), C(n,3), C(n,4) for n = chunk
     const StripInfo* strips;    // split: strips summed by line interpolation, or null
     const int32_t* n_bad;       // strips that are not
+    double2* parts;             // plain: segment sums [segment][record], or null
+    int64_t parts_stride;       // records per segment
 };
 
 // Host launchers (defined in bp_kernels.hip).  `grid` is the number of
@@ -307,7 +317,7 @@ hipError_t launch_pulse_orbit(const Orbit& orbit, double t0, double dt, int na, 
 hipError_t launch_clear(int32_t* words, int n, hipStream_t stream);
 hipError_t launch_geometry(const GeomArgs& args, int grid, hipStream_t stream);
 hipError_t launch_fit(const GeomArgs& args, int grid, hipStream_t stream);
-hipError_t launch_sum_plain(const SumArgs& args, int width, int grid, hipStream_t stream);
+hipError_t launch_sum_plain(const SumArgs& args, int width, int grid, int segs, hipStream_t stream);
 hipError_t launch_sum_split(const SumArgs& args, int width, int grid, bool staged, bool pair,
                             hipStream_t stream);
 int sum_blocks_per_cu(int precision, int width, bool staged, bool pair);
@@ -325,7 +335,7 @@ hipError_t launch_strips(const LineArgs& a, int width, bool last, hipStream_t st
 hipError_t launch_band_window(const PixGeom* geom, int64_t length, int64_t width, int band_rows,
                               int64_t n_bands, int32_t* win, hipStream_t stream);
 // Host-side handle of a kernel (0 geometry, 4 geometry for generic DEMs,
-// 1 plain sum, 2 split sum, 3 fit),
+// 1 plain sum, 5 its segments' total, 2 split sum, 3 fit),
 // as graph kernel nodes report it.
 const void* kernel_fn(int which, int width, bool staged, bool pair);
 

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <limits.h>
 
+#include <algorithm>
 #include <utility>
 
 #include "bp_device.h"
@@ -425,6 +426,11 @@ __device__ inline void for_each_tile(const BatchHeader* batch, Body&& body)
 // kExact: 2 * halfwidth == W, so no tap lies past the half width.
 // `tab2` is the table in LDS or in global memory: each caller passes one of
 // the two, so that the reads compile to LDS or global loads.
+//
+// The sum runs in segments of kPlainSeg pulses (absolute multiples), each
+// segment's sum added to the pixel's in order: batches too small to fill the
+// chip give every segment its own wavefront (`seg` >= 0), which leaves its
+// segment's sum in a.parts for plain_total_kernel to add in the same order.
 // How far the cubic may be off the delay (cycles): the phase's own rounding, a
 // few ulp of fc tau, or 6e-9 rad.
 constexpr double kCubicUlps = 8. / 9007199254740992.;
@@ -433,25 +439,48 @@ constexpr double kCubicTol = 1e-9;
 // good to 2e-8 at the chunk's end (eps^2 / 2 times 64^3 / 6).
 constexpr double kCubicEps = 9e-7;
 
+// One lane's pixel of a plain-sum wavefront tile and the pulses [kw0, kw1) the
+// wavefront's pixels integrate.
+struct PlainPixel {
+    PixGeom g;
+    int64_t pix, tile;
+    bool valid, ok;
+    int ks, ke, kw0, kw1;
+};
+
+__device__ inline PlainPixel plain_pixel(const SumArgs& a, const OutDesc& od, int64_t tile, int lane)
+{
+    PlainPixel p;
+    int64_t row = 0, col = 0;
+    p.tile = tile;
+    p.valid = tile_pixel(od.map, tile, lane, 0, &row, &col);
+    p.pix = row * od.map.width + col;
+    if (p.valid) p.g = a.geom[od.rec_base + p.pix];
+    p.ok = p.valid && p.g.status == kPixOk;
+    p.ks = p.ok ? p.g.kstart : INT_MAX;
+    p.ke = p.ok ? p.g.kstop : INT_MIN;
+    p.kw0 = __builtin_amdgcn_readfirstlane(wave_min_i(p.ks));
+    p.kw1 = __builtin_amdgcn_readfirstlane(wave_max_i(p.ke));
+    return p;
+}
+
 template<int W, bool kExact>
 __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const OutDesc& od,
-                                  int64_t tile, int lane)
+                                  const PlainPixel& px, int seg, int lane)
 {
-    int64_t row = 0, col = 0;
-    const bool valid = tile_pixel(od.map, tile, lane, 0, &row, &col);
-    const int64_t pix = row * od.map.width + col;
-
-    PixGeom g;
-    if (valid) g = a.geom[od.rec_base + pix];
-    const bool ok = valid && g.status == kPixOk;
-    const int ks = ok ? g.kstart : INT_MAX;
-    const int ke = ok ? g.kstop : INT_MIN;
-    const int kw0 = __builtin_amdgcn_readfirstlane(wave_min_i(ks));
-    const int kw1 = __builtin_amdgcn_readfirstlane(wave_max_i(ke));
+    const bool ok = px.ok;
+    const PixGeom& g = px.g;
+    const int ks = px.ks, ke = px.ke;
+    const int kw0 = seg < 0 ? px.kw0 : max(px.kw0, seg * kPlainSeg);
+    const int kw1 = seg < 0 ? px.kw1 : min(px.kw1, (seg + 1) * kPlainSeg);
     const V3 x{g.x[0], g.x[1], g.x[2]};
     const double tau_atm = ok ? g.tau_atm : 0.;
-    const double nr_d = (double)a.nr;
+    // tap m's table offset in scalar registers: 16 vector ones more would spill
+    const double nr_d = readlane_f64((double)a.nr, 0);
     const double rdx = (double)a.rdx;
+    double mrdx[W];
+#pragma unroll
+    for (int m = 0; m < W; ++m) mrdx[m] = readlane_f64((double)m * rdx, 0);  // exact
     const double an_max = a.halfwidth * rdx;
     const int ntab = a.ntab;
 
@@ -471,11 +500,11 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
     // adds pulse k's sample at range bin u times the phasor cs + i sn
     auto add = [&](int k, double u, double cs, double sn) {
         const double low = ((W % 2 == 0) ? ceil(u) : round(u)) - (double)(W / 2);
-        const double a0 = (low - u) * rdx;
+        const double x0 = low - u;
         float w[W];
 #pragma unroll
         for (int m = 0; m < W; ++m) {
-            const double am = a0 + (double)m * rdx;  // m * rdx exact
+            const double am = fma(x0, rdx, mrdx[m]);
             // only the end taps can reach past a half width below W / 2
             w[m] = (!kExact && (m == 0 || m == W - 1))
                        ? tab_weight<true>(tab2, ntab, an_max, am)
@@ -523,7 +552,14 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
     // The chunks begin at multiples of kPlainChunk and the choice is the
     // pixel's own, so that its values do not depend on the pixels that share
     // its wavefront.
+    double tot_re = 0., tot_im = 0.;
+    auto end_segment = [&]() {
+        tot_re += acc_re;
+        tot_im += acc_im;
+        acc_re = acc_im = 0.;
+    };
     for (int k = kw0 / kPlainChunk * kPlainChunk; k < kw1; k += kPlainChunk) {
+        if (k % kPlainSeg == 0) end_segment();
         bool fast = false;
         if ((word(k) & kPosNone) == 0) {
             const Newton3 c = newton3(delay(k + kPlainNode[0]), delay(k + kPlainNode[1]),
@@ -596,9 +632,20 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
             add(i, (tau - a.swst) * a.inv_dtau, cs, sn);
         }
     }
+    // found again here, so that it holds no registers in the sum
+    int end_lane = lane;
+    asm volatile("" : "+v"(end_lane));
+    int64_t row = 0, col = 0;
+    const bool valid = tile_pixel(od.map, px.tile, end_lane, 0, &row, &col);
+    const int64_t pix = row * od.map.width + col;
+    if (seg >= 0) {
+        if (valid) a.parts[seg * a.parts_stride + od.rec_base + pix] = make_double2(acc_re, acc_im);
+        return;
+    }
+    end_segment();
     if (valid) {
         const float nanf_ = __builtin_nanf("");
-        od.out[pix] = ok ? make_float2((float)acc_re, (float)acc_im) : make_float2(nanf_, nanf_);
+        od.out[pix] = ok ? make_float2((float)tot_re, (float)tot_im) : make_float2(nanf_, nanf_);
     }
 }
 
@@ -614,31 +661,60 @@ void sum_plain_kernel(SumArgs a)
 {
     const int64_t ng = uniform64(a.batch->n_groups);
     if ((int64_t)blockIdx.x >= ng) return;
+    const OutDesc* grids = batch_grids(a.batch);
+    const int n_grids = __builtin_amdgcn_readfirstlane(a.batch->n_grids);
+    const int64_t n_seq = uniform64(a.batch->n_seq);
+    const int seg = __builtin_amdgcn_readfirstlane(a.batch->plain_segs) > 0 ? (int)blockIdx.y : -1;
+    int lane;
+    const int64_t gseq = group_tile(blockIdx.x, ng, &lane);
+    const bool in_seq = gseq < n_seq;
+    const OutDesc d = load_desc(grids, in_seq ? find_grid(grids, n_grids, gseq) : 0);
+    const PlainPixel px = plain_pixel(a, d, in_seq ? gseq - d.seq_base : d.map.n_tiles, lane);
+    // a segment that none of the workgroup's pixels integrates
+    if (seg >= 0 && !__syncthreads_or(px.kw0 < (seg + 1) * kPlainSeg && px.kw1 > seg * kPlainSeg))
+        return;
     extern __shared__ double2 s_tab2[];
     const bool tab_in_lds = a.ntab <= kMaxTab2Lds;
     if (tab_in_lds)
         for (int i = threadIdx.x; i < a.ntab; i += blockDim.x) s_tab2[i] = a.tab2[i];
     __syncthreads();
+    if (!in_seq) return;
+    if (tab_in_lds) {
+        if (a.exact_width)
+            plain_tile<W, true>(a, s_tab2, d, px, seg, lane);
+        else
+            plain_tile<W, false>(a, s_tab2, d, px, seg, lane);
+    } else {
+        if (a.exact_width)
+            plain_tile<W, true>(a, a.tab2, d, px, seg, lane);
+        else
+            plain_tile<W, false>(a, a.tab2, d, px, seg, lane);
+    }
+}
+
+// The segments' sums of each pixel, in pulse order (256 threads per group of
+// four tiles, as the sum).
+__global__ __launch_bounds__(256) void plain_total_kernel(SumArgs a)
+{
+    const int64_t ng = uniform64(a.batch->n_groups);
+    if ((int64_t)blockIdx.x >= ng || __builtin_amdgcn_readfirstlane(a.batch->plain_segs) == 0) return;
     const OutDesc* grids = batch_grids(a.batch);
-    const int n_grids = __builtin_amdgcn_readfirstlane(a.batch->n_grids);
-    const int64_t n_seq = uniform64(a.batch->n_seq);
     int lane;
     const int64_t gseq = group_tile(blockIdx.x, ng, &lane);
-    if (gseq < n_seq) {
-        const OutDesc d = load_desc(grids, find_grid(grids, n_grids, gseq));
-        const int64_t t = gseq - d.seq_base;
-        if (tab_in_lds) {
-            if (a.exact_width)
-                plain_tile<W, true>(a, s_tab2, d, t, lane);
-            else
-                plain_tile<W, false>(a, s_tab2, d, t, lane);
-        } else {
-            if (a.exact_width)
-                plain_tile<W, true>(a, a.tab2, d, t, lane);
-            else
-                plain_tile<W, false>(a, a.tab2, d, t, lane);
+    if (gseq >= uniform64(a.batch->n_seq)) return;
+    const OutDesc d =
+        load_desc(grids, find_grid(grids, __builtin_amdgcn_readfirstlane(a.batch->n_grids), gseq));
+    const PlainPixel px = plain_pixel(a, d, gseq - d.seq_base, lane);
+    if (!px.valid) return;
+    double re = 0., im = 0.;
+    if (px.ok && px.ke > px.ks)
+        for (int s = px.ks / kPlainSeg; s <= (px.ke - 1) / kPlainSeg; ++s) {
+            const double2 v = a.parts[s * a.parts_stride + d.rec_base + px.pix];
+            re += v.x;
+            im += v.y;
         }
-    }
+    const float nanf_ = __builtin_nanf("");
+    d.out[px.pix] = px.ok ? make_float2((float)re, (float)im) : make_float2(nanf_, nanf_);
 }
 
 // Split-precision coherent sum of one wavefront tile.
@@ -1501,13 +1577,14 @@ size_t plain_lds(int ntab) { return ntab <= kMaxTab2Lds ? sizeof(double2) * ntab
 }  // namespace
 
 // Host-side handle of a kernel (0 geometry, 4 geometry for generic DEMs,
-// 1 plain sum, 2 split sum, 3 fit), as graph kernel nodes report it; null for
+// 1 plain sum, 5 its segments' total, 2 split sum, 3 fit), as graph kernel nodes report it; null for
 // a width or variant that is not built.
 const void* kernel_fn(int which, int width, bool staged, bool pair)
 {
     switch (which) {
     case 0: return reinterpret_cast<const void*>(&geometry_kernel<false>);
     case 4: return reinterpret_cast<const void*>(&geometry_kernel<true>);
+    case 5: return reinterpret_cast<const void*>(&plain_total_kernel);
     case 3: return reinterpret_cast<const void*>(&fit_kernel);
     case 1: return width_ok(width) ? plain_fn(width, Widths{}) : nullptr;
     default:
@@ -1522,13 +1599,18 @@ const void* kernel_fn(int which, int width, bool staged, bool pair)
     }
 }
 
-hipError_t launch_sum_plain(const SumArgs& args, int width, int grid, hipStream_t stream)
+hipError_t launch_sum_plain(const SumArgs& args, int width, int grid, int segs, hipStream_t stream)
 {
     if (grid <= 0) return hipSuccess;
     const void* fn = kernel_fn(1, width, false, false);
     if (fn == nullptr) return hipErrorInvalidValue;
     void* kargs[] = {const_cast<SumArgs*>(&args)};
-    return hipLaunchKernel(fn, dim3(grid), dim3(256), kargs, plain_lds(args.ntab), stream);
+    hipError_t e = hipLaunchKernel(fn, dim3(grid, std::max(segs, 1)), dim3(256), kargs,
+                                   plain_lds(args.ntab), stream);
+    if (e == hipSuccess && args.parts != nullptr)
+        e = hipLaunchKernel(kernel_fn(5, width, false, false), dim3(grid), dim3(256), kargs, 0,
+                            stream);
+    return e;
 }
 
 // Workgroups one CU can hold for the chosen sum kernel (256 threads for the

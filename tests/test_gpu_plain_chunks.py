@@ -60,3 +60,27 @@ def test_windows_inside_chunks(torch_gpu, na):
 @pytest.mark.parametrize("prf", [100.0, 700.0, 3000.0])
 def test_short_ranges(torch_gpu, prf):
     _check(330, 6.0, altitude=3000.0, speed=120.0, prf=prf, r0=5000.0)
+
+
+def test_segments_and_whole_windows_agree(torch_gpu):
+    """A grid of more wavefronts than get segments of their own, and its first
+    rows alone, which are summed by segments: the same to the bit."""
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import KnabKernel, LUT2d, TabulatedKernelF32
+    from isce3_amd.focus import backproject
+    from isce3_amd.geometry import DEMInterpolator
+    na, nr, rows, cols = 1500, 1060, 1040, 1030
+    orb = sim.straight_orbit()
+    in_grid = sim._grid(-0.5 * na / sim.PRF, sim.PRF, sim.R0, sim.DR, na, nr)
+    rng = np.random.default_rng(1)
+    raw = (rng.standard_normal((na, nr)) + 1j * rng.standard_normal((na, nr))).astype(np.complex64)
+    kernel = TabulatedKernelF32(KnabKernel(8.0, 0.8), 2048)
+    outs = []
+    for n in (rows, 33):
+        grid = sim._grid(-0.5 * rows / sim.PRF, sim.PRF, sim.R0 + 12 * sim.DR, sim.DR, n, cols)
+        out = np.empty(grid.shape, np.complex64)
+        backproject(out, RadarGeometry(grid, orb, LUT2d()), raw, RadarGeometry(in_grid, orb, LUT2d()),
+                    DEMInterpolator(50.0), sim.FC, 40.0, kernel, "nodelay", precision="plain")
+        outs.append(out)
+    np.testing.assert_array_equal(outs[0][:33], outs[1])
