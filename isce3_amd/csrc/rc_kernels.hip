@@ -125,6 +125,22 @@ __device__ inline void dft<16>(float2 (&v)[16])
         for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = t[4 * k1 + k2];
 }
 
+// As twiddle<16>, with W^t .. W^3t and W^4t, W^8t, W^12t from the table and one
+// product for each of the others.
+__device__ inline void twiddle16_table(float2 (&v)[16], const float2* __restrict__ tw, int t)
+{
+    const float2 lo[4] = {make_float2(1.f, 0.f), tw[t], tw[2 * t], tw[3 * t]};
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        const float2 hi = tw[4 * h * t];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (h == 0 && r == 0) continue;
+            v[4 * h + r] = cmul(v[4 * h + r], r == 0 ? hi : (h == 0 ? lo[r] : cmul(hi, lo[r])));
+        }
+    }
+}
+
 // v[r] *= W^(r t) with W = exp(-2 pi i / L), from the table tw[k] = W^k.
 template<int R>
 __device__ inline void twiddle(float2 (&v)[R], const float2* __restrict__ tw, int t)
@@ -163,54 +179,8 @@ __device__ inline void twiddle(float2 (&v)[R], const float2* __restrict__ tw, in
     for (int r = 1; r < R; ++r) v[r] = cmul(v[r], w[r]);
 }
 
-// One Stockham pass of radix R at sub-transform size Ns over L values in
-// padded LDS, T = L / 16 threads, each taking 16 / R butterflies.
-template<int R, int L>
-__device__ inline void stockham_pass(float2* s, int Ns, const float2* __restrict__ tw)
-{
-    constexpr int T = L / 16;
-    constexpr int NB = L / R;
-    constexpr int Q = NB / T;
-    float2 v[Q][R];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int j = threadIdx.x + q * T;
-#pragma unroll
-        for (int r = 0; r < R; ++r) v[q][r] = s[pad(j + r * NB)];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int j = threadIdx.x + q * T;
-        const int k = j & (Ns - 1);
-        if (Ns > 1) twiddle<R>(v[q], tw, k * (L / (Ns * R)));
-        dft<R>(v[q]);
-        const int base = (j - k) * R + k;
-#pragma unroll
-        for (int r = 0; r < R; ++r) s[pad(base + r * Ns)] = v[q][r];
-    }
-    __syncthreads();
-}
-
-// Forward FFT of L = 2^LOG2L (10 <= LOG2L <= 14) values in padded LDS.
-template<int LOG2L>
-__device__ inline void fft(float2* s, const float2* __restrict__ tw)
-{
-    constexpr int L = 1 << LOG2L;
-    constexpr int NR16 = LOG2L / 4;
-    constexpr int REM = LOG2L % 4;
-    int Ns = 1;
-#pragma unroll
-    for (int p = 0; p < NR16; ++p) {
-        stockham_pass<16, L>(s, Ns, tw);
-        Ns *= 16;
-    }
-    if (REM == 1) stockham_pass<2, L>(s, Ns, tw);
-    if (REM == 2) stockham_pass<4, L>(s, Ns, tw);
-    if (REM == 3) stockham_pass<8, L>(s, Ns, tw);
-}
-
-// A Stockham pass split into its parts so that the first pass can read from
+// A Stockham pass of radix R at sub-transform size Ns, T = L / 16 threads, each
+// taking 16 / R butterflies, split into its parts so that the first pass can read from
 // global memory and the last pass of the forward transform can hand its
 // outputs to the first pass of the inverse transform in registers.  Thread t
 // holds butterflies j = t + q T (q < 16 / R), element r of butterfly j being
@@ -415,21 +385,19 @@ __device__ inline void dft<32>(float2 (&v)[32])
     }
 }
 
-// v[k] *= W_L^(n k) for k < 32 from the table tw[j] = W_L^j, j < L: three
-// reads (W^n, W^4n, W^16n) and at most four products per factor.
+// v[k] *= W_L^(n k) for k < 32 from the table tw[j] = W_L^j, j < L: ten reads
+// (W^n .. W^3n and W^4n, W^8n .. W^28n) and one product for each other factor.
 __device__ inline void twiddle32(float2 (&v)[32], const float2* __restrict__ tw, int n)
 {
-    const float2 w1 = tw[n], w4 = tw[4 * n], w16 = tw[16 * n];
-    const float2 w2 = cmul(w1, w1), w3 = cmul(w2, w1);
-    const float2 w8 = cmul(w4, w4), w12 = cmul(w8, w4);
-    const float2 lo[4] = {make_float2(1.f, 0.f), w1, w2, w3};
-    const float2 mid[4] = {make_float2(1.f, 0.f), w4, w8, w12};
+    const float2 lo[4] = {make_float2(1.f, 0.f), tw[n], tw[2 * n], tw[3 * n]};
 #pragma unroll
-    for (int k = 1; k < 32; ++k) {
-        float2 w = mid[(k >> 2) & 3];
-        if (k & 3) w = (k >> 2) & 3 ? cmul(w, lo[k & 3]) : lo[k & 3];
-        if (k & 16) w = cmul(w, w16);
-        v[k] = cmul(v[k], w);
+    for (int h = 0; h < 8; ++h) {
+        const float2 hi = tw[4 * h * n];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (h == 0 && r == 0) continue;
+            v[4 * h + r] = cmul(v[4 * h + r], r == 0 ? hi : (h == 0 ? lo[r] : cmul(hi, lo[r])));
+        }
     }
 }
 
@@ -453,22 +421,77 @@ __global__ __launch_bounds__(256) void col_fwd_kernel(ConvArgs a)
     for (int k1 = 0; k1 < 32; ++k1) y[(int64_t)k1 * L2 + n2] = v[k1];
 }
 
+// Rows of the four steps: as the passes of conv_kernel (transform, product
+// and second transform, with the row's ends and the product in registers), with
+// the radix-16 passes' factors read from the table: the second transform
+// ends in two such passes where separate transforms ended in one, and factors
+// of two products left an error of 2.8e-7 (two separate transforms: 2.6e-7; factors from
+// the table here and in the columns: 2.3e-7).
+// Bound by LDS traffic and barriers: six passes through LDS instead of ten,
+// 300 pulses of 30000 samples (2^15 points) 105 us instead of 134 for all three
+// kernels (111 with the columns' factors from the table).
 template<int LOG2L2>
 __global__ __launch_bounds__((1 << LOG2L2) / 16) void row_kernel(ConvArgs a)
 {
     constexpr int L2 = 1 << LOG2L2;
     constexpr int T = L2 / 16;
+    constexpr int Rl = LastRadix<LOG2L2 % 4>::R;
+    constexpr int N16 = (LOG2L2 - (Rl == 16 ? 4 : 0)) / 4;
     __shared__ float2 s[L2 + L2 / 16];
     const int k1 = blockIdx.x;
     float2* row = a.work + (int64_t)blockIdx.y * (32 * L2) + (int64_t)k1 * L2;
-    for (int i = threadIdx.x; i < L2; i += T) s[pad(i)] = row[i];
-    __syncthreads();
-    fft<LOG2L2>(s, a.tw2);
-    const float2* h = a.H + (int64_t)k1 * L2;   // permuted spectrum: bin k1 + 32 k2 at [k1][k2]
-    for (int i = threadIdx.x; i < L2; i += T) s[pad(i)] = conjf2(cmul(s[pad(i)], h[i]));
-    __syncthreads();
-    fft<LOG2L2>(s, a.tw2);
-    for (int i = threadIdx.x; i < L2; i += T) row[i] = s[pad(i)];
+    auto pass16 = [&](Regs<16, L2>& d, int Ns) {
+        if (Ns > 1) twiddle16_table(d.v[0], a.tw2, (threadIdx.x & (Ns - 1)) * (T / Ns));
+        dft<16>(d.v[0]);
+    };
+    auto pass16_lds = [&](int Ns) {
+        Regs<16, L2> d;
+        pass_load_lds(d, s);
+        __syncthreads();
+        pass16(d, Ns);
+        pass_store_lds(d, s, Ns);
+        __syncthreads();
+    };
+    {
+        Regs<16, L2> d;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) d.v[0][r] = row[threadIdx.x + r * T];
+        pass16(d, 1);
+        pass_store_lds(d, s, 1);
+        __syncthreads();
+    }
+    int Ns = 16;
+#pragma unroll
+    for (int p = 1; p < N16; ++p, Ns *= 16) pass16_lds(Ns);
+    {
+        Regs<Rl, L2> d;
+        pass_load_lds(d, s);
+        __syncthreads();
+        if constexpr (Rl == 16)
+            pass16(d, Ns);
+        else
+            pass_compute(d, Ns, a.tw2);
+        const float2* h = a.H + (int64_t)k1 * L2;   // permuted spectrum: bin k1 + 32 k2 at [k1][k2]
+#pragma unroll
+        for (int q = 0; q < d.Q; ++q) {
+            const int j = threadIdx.x + q * T;
+#pragma unroll
+            for (int r = 0; r < Rl; ++r) d.v[q][r] = conjf2(cmul(d.v[q][r], h[j + r * Ns]));
+        }
+        pass_compute(d, 1, a.tw2);
+        pass_store_lds(d, s, 1);
+        __syncthreads();
+    }
+    Ns = Rl;
+#pragma unroll
+    for (int p = 0; p + 1 < N16; ++p, Ns *= 16) pass16_lds(Ns);
+    {
+        Regs<16, L2> d;
+        pass_load_lds(d, s);
+        pass16(d, Ns);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) row[threadIdx.x + r * T] = d.v[0][r];
+    }
 }
 
 template<int LOG2L2>

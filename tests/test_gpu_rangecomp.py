@@ -209,3 +209,25 @@ def test_long_pulses_more_than_one_work_batch(torch_gpu):
         e = rel_err(y[i], ref[i])
         print(f"[rangecomp seam] pulse {r} rel={e:.2e}", flush=True)
         assert e <= REL
+
+
+@pytest.mark.parametrize("mode,m,nin,length", [
+    ("valid", 9000, 32768, 1 << 15), ("valid", 9000, 32769, 1 << 16), ("valid", 32768, 32768, 1 << 15),
+    ("valid", 8195, 8200, 1 << 15), ("same", 12000, 26768, 1 << 15), ("same", 12001, 26768, 1 << 15),
+    ("same", 12001, 26769, 1 << 16), ("full", 12000, 26768, 1 << 16), ("valid", 33000, 20000, 1 << 16)])
+def test_four_step_lengths_wrap_only_unwanted_samples(torch_gpu, mode, m, nin, length):
+    """Transforms shorter than the full convolution, at the lengths where its
+    tail just misses the wanted samples, and those that keep the full length
+    (full mode, chirps longer than the pulse)."""
+    from isce3_amd.focus import RangeComp
+    rng = np.random.default_rng(nin + m)
+    chirp = np.exp(1j * np.pi * 1e-5 * (np.arange(m) - m / 2) ** 2).astype(np.complex64)
+    x = (rng.standard_normal((2, nin)) + 1j * rng.standard_normal((2, nin))).astype(np.complex64)
+    rc = RangeComp(chirp, nin, maxbatch=2, mode=RangeComp.Mode[mode.capitalize()])
+    print(f"[rangecomp wrap] mode={mode} nin={nin} m={m} plan={rc.plan}", flush=True)
+    if rc.plan[0] == "four-step":
+        assert rc.plan[1] == length
+    y = np.zeros((2, rc.output_size), np.complex64)
+    rc.rangecompress(y, x)
+    ref = rco.rangecompress(chirp, x, MODES[mode], "fp64")
+    assert rel_err(y, ref) <= REL
