@@ -1209,6 +1209,7 @@ void set_lines(Step& sp, const LinePlan& p, const Scratch& sc, const CallArgs& a
     la.s_end = group;
     la.q_begin = INT32_MIN;
     la.q_end = INT32_MAX;
+    la.few = n <= bp::kFewStrips ? 1 : 0;
     bp::line_place(la, static_cast<unsigned char*>(sc.lines.ptr), group);
     sp.lines = true;
     sp.n_strips = n;
@@ -2017,8 +2018,10 @@ int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
     bp_context* c = sc->ctx;
     Step sp;
     build_step(sp, sc->st, sc->sc, sc->args, sc->width, o, c->n_cu);
-    if (sc->lines.on && o.lane_rows == 2 && !o.staged)
+    if (sc->lines.on && o.lane_rows == 2 && !o.staged) {
         set_lines(sp, sc->lines, sc->sc, sc->args, sc->line_strips, sc->line_group);
+        if (sp.la.few == 0) sp.la.few = 2;   // replayed with any count up to line_strips
+    }
     if (sc->part_records > 0) {
         sp.sa.parts = static_cast<double2*>(sc->sc.parts.ptr);
         sp.sa.parts_stride = sc->part_records;
@@ -2097,7 +2100,8 @@ int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
     }
     const size_t groups =
         sp.lines ? (size_t)((sp.n_strips + sp.group_strips - 1) / sp.group_strips) : 0;
-    const size_t want = 2 + (total_fn ? 1 : 0) + (sp.lines ? 1 + 4 * groups : 0);
+    const size_t per_group = sp.lines && sp.la.few == 2 ? 5 : 4;
+    const size_t want = 2 + (total_fn ? 1 : 0) + (sp.lines ? 1 + per_group * groups : 0);
     if (out->nodes.size() != want) {
         (void)hipGraphDestroy(g);
         return fail(BP_ERR_HIP, "captured step is missing its kernel nodes");

@@ -250,6 +250,8 @@ struct LineArgs {
     unsigned long long* cross;           // [strip][slot][8 nodes]
     float farrow[kLineDegree + 1][kLineTaps];
     float w_in[kEndDegree + 1], w_out[kEndDegree + 1];
+    int32_t few;                // lines kernel: 0 for many strips, 1 for up to
+                                // kFewStrips, 2 chosen by the batch's count
 };
 
 __host__ __device__ inline const OutDesc* batch_grids(const BatchHeader* b)
@@ -321,9 +323,15 @@ hipError_t launch_sum_plain(const SumArgs& args, int width, int grid, int segs, 
 hipError_t launch_sum_split(const SumArgs& args, int width, int grid, bool staged, bool pair,
                             hipStream_t stream);
 int sum_blocks_per_cu(int precision, int width, bool staged, bool pair);
+// Strips up to which a segment of a line group gets four wavefronts instead of
+// one.  Whole calls on tiles of 1, 4, 16 and 25 strips (32, 128, 256 and 300
+// pixels square, 4,000 pulses): 221, 302, 394 and 461 us with four, 251, 356, 400
+// and 443 us with one.
+constexpr int kFewStrips = 16;
+
 // Line-interpolated split sum (bp_lines.hip): workspace bytes per strip and
 // its placement, kernels and their grids.
-enum LineKernel : int { kLineFit = 0, kLineNodes, kLineLines, kLineEnds, kLineSum };
+enum LineKernel : int { kLineFit = 0, kLineNodes, kLineLines, kLineFew, kLineEnds, kLineSum };
 size_t line_strip_bytes(int slots, int n_sums);
 size_t line_carry_bytes();
 void line_place(LineArgs& a, unsigned char* ws, int64_t n_strips);

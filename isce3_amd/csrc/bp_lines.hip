@@ -604,9 +604,10 @@ __device__ inline void load_end_taps(const char* row, uint32_t off, float2 (&x)[
 
 // Chunks [c0, c1) of a group of lines: interpolated node sums and the
 // corrections of the pulses at which a line's cell is not the reference's.
-template<int W, int N, bool kSlopes>
+// Every `step`th; `add` takes each one's sums.
+template<int W, int N, bool kSlopes, class Add>
 __device__ inline void line_chunks(const LineArgs& a, const Strip& st, const StripInfo& in, int g,
-                                   int c0, int c1, int64_t ws, int lane, Sum64 (&acc)[kGroupLines])
+                                   int c0, int c1, int step, int64_t ws, int lane, Add&& add)
 {
     constexpr int G = kGroupLines;
     const int col = min(lane, st.cols - 1);
@@ -646,7 +647,7 @@ __device__ inline void line_chunks(const LineArgs& a, const Strip& st, const Str
     }
     nlo = __builtin_amdgcn_readfirstlane(nlo);
     nhi = __builtin_amdgcn_readfirstlane(nhi);
-    for (int c = c0; c < c1; ++c) {
+    for (int c = c0; c < c1; c += step) {
         const int first = (in.slot0 + c) << a.chunk_log2;
         if (first < a.q_begin || first >= a.q_end) continue;
         // the records are read anew for every chunk (kept in registers they
@@ -755,11 +756,7 @@ __device__ inline void line_chunks(const LineArgs& a, const Strip& st, const Str
                 }
             }
         }
-#pragma unroll
-        for (int i = 0; i < G; ++i) {
-            acc[i].x += (double)cre[i];
-            acc[i].y += (double)cim[i];
-        }
+        add(c, cre, cim);
     }
 }
 
@@ -863,6 +860,23 @@ __device__ inline void line_ends(const LineArgs& a, const Strip& st, const Strip
     }
 }
 
+template<int W, class Add>
+__device__ inline void any_chunks(const LineArgs& a, const Strip& st, const StripInfo& in, int g,
+                                  int c0, int c1, int step, int64_t ws, int lane, Add&& add)
+{
+    if (in.slopes) {
+        if (st.h <= 32)
+            line_chunks<W, 6, true>(a, st, in, g, c0, c1, step, ws, lane, add);
+        else
+            line_chunks<W, 8, true>(a, st, in, g, c0, c1, step, ws, lane, add);
+    } else {
+        if (st.h <= 32)
+            line_chunks<W, 6, false>(a, st, in, g, c0, c1, step, ws, lane, add);
+        else
+            line_chunks<W, 8, false>(a, st, in, g, c0, c1, step, ws, lane, add);
+    }
+}
+
 // One wavefront per group of kGroupLines lines and segment: a quarter of the
 // strip's chunks (strip_lines_kernel) or one of the aperture's ends
 // (strip_ends_kernel).  Workgroups of one wavefront: the groups' work differs
@@ -901,17 +915,14 @@ __device__ inline void group_sums(const LineArgs& a)
         line_ends<W>(a, st, si, g, seg == kCoreSegs, lane, acc);
     } else {
         const int c0 = seg * si.nslots / kCoreSegs, c1 = (seg + 1) * si.nslots / kCoreSegs;
-        if (si.slopes) {
-            if (st.h <= 32)
-                line_chunks<W, 6, true>(a, st, si, g, c0, c1, ws, lane, acc);
-            else
-                line_chunks<W, 8, true>(a, st, si, g, c0, c1, ws, lane, acc);
-        } else {
-            if (st.h <= 32)
-                line_chunks<W, 6, false>(a, st, si, g, c0, c1, ws, lane, acc);
-            else
-                line_chunks<W, 8, false>(a, st, si, g, c0, c1, ws, lane, acc);
-        }
+        auto add = [&](int, const float (&cre)[kGroupLines], const float (&cim)[kGroupLines]) {
+#pragma unroll
+            for (int i = 0; i < kGroupLines; ++i) {
+                acc[i].x += (double)cre[i];
+                acc[i].y += (double)cim[i];
+            }
+        };
+        any_chunks<W>(a, st, si, g, c0, c1, 1, ws, lane, add);
     }
     if (a.carry != nullptr) {
 #pragma unroll
@@ -926,7 +937,67 @@ template<int W>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
 void strip_lines_kernel(LineArgs a)
 {
+    if (a.few == 2 && uniform64(a.batch->n_strips) <= kFewStrips) return;
     group_sums<W, false>(a);
+}
+
+// As strip_lines_kernel, with a workgroup of four wavefronts per segment and
+// group: each takes every fourth chunk and leaves its sums in LDS, then line i's
+// are added by wavefront i in the order of the chunks, so that the sums do not
+// depend on which kernel ran.  A single strip is 32 to 64 segments, each of 16
+// chunks of 8,000 cycles of issue one after the other: 54 us for 32 x 32 pixels
+// of 4,000 pulses, 27 us here.  Few wavefronts are in flight, so each has the
+// registers it needs (two per SIMD; at four they spill: 31 us).
+template<int W>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void strip_few_kernel(LineArgs a)
+{
+    constexpr int kRound = 20;   // chunks held at once
+    static_assert(kGroupLines == 4, "a wavefront per line");
+    __shared__ float2 s_sum[kRound][kGroupLines][64];
+    const int64_t n_strips = uniform64(a.batch->n_strips);
+    if (a.few == 2 && n_strips > kFewStrips) return;
+    const int64_t end = min(a.s_end, n_strips);
+    const int64_t item = blockIdx.x;
+    const int64_t ws = item / (kCoreSegs * kMaxGroups);
+    const int rest = (int)(item - ws * (kCoreSegs * kMaxGroups));
+    const int seg = rest / kMaxGroups, g = rest % kMaxGroups;
+    const int64_t t = a.s_begin + ws;
+    if (t >= end) return;
+    const OutDesc* grids = batch_grids(a.batch);
+    const OutDesc d =
+        load_desc(grids, find_strip_grid(grids, __builtin_amdgcn_readfirstlane(a.batch->n_grids), t));
+    const Strip st = load_strip(d, t);
+    const auto* in = uniform_ptr(a.info) + st.info;
+    const StripInfo si{in->k0, in->k1, in->f0, in->f1, in->ok, in->slot0, in->nslots, in->slopes};
+    if (!si.ok || g * kGroupLines >= st.h) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t at = (ws * kSegs + seg) * (kStripLines * 64) + (g * kGroupLines + wave) * 64 + lane;
+    Sum64 acc = make_double2(0., 0.);
+    if (a.carry != nullptr && !a.q_first) acc = a.carry[at];
+    const int c0 = seg * si.nslots / kCoreSegs, c1 = (seg + 1) * si.nslots / kCoreSegs;
+    for (int r0 = c0; r0 < c1; r0 += kRound) {
+        const int r1 = min(c1, r0 + kRound);
+        auto keep = [&](int c, const float (&cre)[kGroupLines], const float (&cim)[kGroupLines]) {
+#pragma unroll
+            for (int i = 0; i < kGroupLines; ++i)
+                s_sum[c - r0][i][lane] = make_float2(cre[i], cim[i]);
+        };
+        any_chunks<W>(a, st, si, g, r0 + wave, r1, kGroupLines, ws, lane, keep);
+        __syncthreads();
+        for (int c = r0; c < r1; ++c) {
+            // chunks of other parts of the pulses were passed over
+            const int first = (si.slot0 + c) << a.chunk_log2;
+            if (first < a.q_begin || first >= a.q_end) continue;
+            const float2 v = s_sum[c - r0][wave][lane];
+            acc.x += (double)v.x;
+            acc.y += (double)v.y;
+        }
+        __syncthreads();
+    }
+    if (a.carry != nullptr) a.carry[at] = acc;
+    a.parts[at] = make_float2((float)acc.x, (float)acc.y);
 }
 
 template<int W>
@@ -995,6 +1066,7 @@ const void* width_fn(int which)
     switch (which) {
     case kLineNodes: return reinterpret_cast<const void*>(&strip_nodes_kernel<W>);
     case kLineLines: return reinterpret_cast<const void*>(&strip_lines_kernel<W>);
+    case kLineFew: return reinterpret_cast<const void*>(&strip_few_kernel<W>);
     case kLineEnds: return reinterpret_cast<const void*>(&strip_ends_kernel<W>);
     case kLineSum: return reinterpret_cast<const void*>(&strip_sum_kernel);
     default: return reinterpret_cast<const void*>(&strip_fit_kernel);
@@ -1015,7 +1087,8 @@ int64_t line_grid(int which, int slots, int64_t n)
     switch (which) {
     case kLineFit: return n;
     case kLineNodes: return (n * slots + kWaves - 1) / kWaves;
-    case kLineLines: return n * kCoreSegs * kMaxGroups;
+    case kLineLines:
+    case kLineFew: return n * kCoreSegs * kMaxGroups;
     case kLineEnds: return n * (kSegs - kCoreSegs) * kMaxGroups;
     default: return n * 4;
     }
@@ -1034,6 +1107,7 @@ hipError_t launch_strips(const LineArgs& a, int width, bool last, hipStream_t st
 {
     void* kargs[] = {const_cast<LineArgs*>(&a)};
     for (int which = kLineNodes; which <= (last ? kLineSum : kLineEnds); ++which) {
+        if (which == (a.few == 0 ? kLineFew : a.few == 1 ? kLineLines : kLineFit)) continue;
         const int64_t grid = line_grid(which, a.slots, a.s_end - a.s_begin);
         if (grid <= 0) continue;
         const void* fn = line_kernel_fn(which, width);

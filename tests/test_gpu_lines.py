@@ -131,3 +131,24 @@ def test_whole_and_band_by_band_agree(torch_gpu):
             assert st["bands"] >= 2
     np.testing.assert_array_equal(outs[1], outs[0])
     np.testing.assert_array_equal(outs[2], outs[0])
+
+
+@pytest.mark.parametrize("width,tropo", [(8, "nodelay"), (9, "tsx")])
+def test_few_and_many_strips_agree(torch_gpu, width, tropo):
+    """The lines kernel of a few strips (four wavefronts per segment) and that of
+    many, on the same strip: a block of 18 strips and its first one alone, the
+    same to the bit."""
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import LUT2d
+    from isce3_amd.focus import backproject
+    orb, in_geom, dem, raw, kernel = _scene(width, relief=100.0 if tropo == "tsx" else 0.0)
+    outs = []
+    for cols, rows in ((64, 64 * 18), (64, 64)):
+        grid = sim._grid(-0.2, sim.PRF, sim.R0 + 40 * sim.DR, sim.DR,
+                         rows, cols)
+        out = np.empty(grid.shape, np.complex64)
+        backproject(out, RadarGeometry(grid, orb, LUT2d()), raw, in_geom, dem, sim.FC, 6.0, kernel,
+                    tropo, precision="split")
+        outs.append(out)
+    np.testing.assert_array_equal(outs[0][:64], outs[1])
