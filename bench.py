@@ -38,6 +38,10 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 FLOPS_PER_UPDATE = 101  # algorithmic flops per pixel-pulse update (FMA = 2)
+# ... and those that the line-interpolated sum executes in place of the 101: per
+# pulse and column 256 for the tap polynomials and 40 for each of 8 node lines,
+# shared by the 64 lines of a strip (kernel width 8; corrections and ends not counted)
+LINE_FLOPS_PER_UPDATE = (256 + 8 * 40) / 64
 PEAK_FP32_TFLOPS = 157.3
 PEAK_FP64_TFLOPS = 78.6
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "sum_split_kernel_two_lines_pmc.md")
@@ -626,10 +630,14 @@ def split_kernel_name(opts) -> str:
     """The coherent-sum kernel the split step ran with these launch options
     (kernel width 8)."""
     staged = bool((opts or {}).get("staged", 0))
-    lanes = (opts or {}).get("lane_rows", 0)
-    pair = not staged and lanes in (0, 2)
-    return (f"sum_split_kernel<8, {'true' if staged else 'false'}, {'true' if pair else 'false'}>"
-            + (" (two output lines per lane)" if pair else ""))
+    if split_by_lines(opts):
+        return "strip_nodes/lines/ends/sum_kernel<8> (64 output lines from 8 node lines)"
+    return f"sum_split_kernel<8, {'true' if staged else 'false'}, false>"
+
+
+def split_by_lines(opts) -> bool:
+    """Whether these launch options let the split sum interpolate between lines."""
+    return not (opts or {}).get("staged", 0) and (opts or {}).get("lane_rows", 0) in (0, 2)
 
 
 def main():
@@ -736,7 +744,9 @@ def main():
     presum_res = None if args.no_presum else run_presum(args, torch, np, dev)
 
     sp, pl = results["split"], results["plain"]
-    achieved = sp["updates"] * FLOPS_PER_UPDATE / (sp["sum_ms"] * 1e-3) / 1e12
+    by_lines = split_by_lines(sp["options"])
+    flops = LINE_FLOPS_PER_UPDATE if by_lines else FLOPS_PER_UPDATE
+    achieved = sp["updates"] * flops / (sp["sum_ms"] * 1e-3) / 1e12
     latency = None
     if serve_res:
         latency = {f"{r['rate_per_s']:g}/s": {"p50_ms": r["split_batched"]["p50_ms"],
@@ -767,7 +777,8 @@ def main():
         "split_over_plain": sp["updates_per_s"] / pl["updates_per_s"],
         "roofline": {"bound": "valu", "kernel": split_kernel_name(sp["options"]),
                      "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_FP32_TFLOPS, "traffic": hbm_bytes_per_launch()},
+                     "frac": achieved / PEAK_FP32_TFLOPS,
+                     "flops_per_update": flops, "traffic": None if by_lines else hbm_bytes_per_launch()},
         "latency": latency,
         "batch": batch,
         "serve": serve_res,

@@ -160,7 +160,11 @@ typedef struct {
                               1 stages each pulse's range window in LDS first */
     int32_t lane_rows;     /* output lines per lane of the split sum: 2 (adjacent lines
                               share their taps; kernel width 8, staged 0 only), 1, or 0 =
-                              2 where offered, else 1 (default) */
+                              2 where offered, else 1 (default).  With 0 or 2, staged
+                              0 and kernel width 8 or 9, strips of up to 64 output
+                              lines are interpolated between node lines where the
+                              geometry allows, and the options above only shape
+                              the sum of the strips that remain */
     int32_t reserved[1];
 } bp_options;
 

@@ -13,7 +13,9 @@ The tunable options are those of ``bp_options`` (include/isce3_amd_backproject.h
     lane_rows      output lines per lane of the split sum (2: adjacent lines
                    share one gather; staged 0 only -- with staged 1 the call
                    raises InvalidArgument and the candidate scores as
-                   infinitely slow)
+                   infinitely slow); with 2 and kernel width 8 or 9 most strips
+                   are interpolated between lines and the other options only
+                   shape what remains
 
 The plain kernel only has ``tile_rows``.  A tuning run times candidates with
 the device-side HIP-event times that every call reports (geometry + sum),

@@ -3,9 +3,11 @@
 //   geometry_kernel     FP64 per-pixel rdr2geo/geo2rdr, CPI window, TSX delay,
 //                       and (split mode) the per-pixel delay polynomial fit
 //   sum_plain_kernel    reference-semantics coherent sum, FP64 delay & phase
+//   plain_total_kernel  its segments' sums of small grids
 //   sum_split_kernel    split-precision coherent sum: FP64 polynomial phase,
 //                       FP32 range-bin delta, polyphase weights from LDS,
 //                       FP32 complex MACs with Kahan-compensated chunk sums
+//                       (strips that bp_lines.hip leaves, and other widths)
 #include <hip/hip_runtime.h>
 #include <limits.h>
 
@@ -422,7 +424,7 @@ __device__ inline void for_each_tile(const BatchHeader* batch, Body&& body)
 // tap m's table coordinate is then x0 * float(1/dx) + m * float(1/dx) (the
 // reference rounds (x0 + m) * float(1/dx) once instead of twice: the index
 // and fraction agree to an ulp of the coordinate).  The phase 2 pi fc tau
-// comes from sincos_turns of fc tau in FP64.
+// comes from sincos_turns of fc tau in FP64, per chunk or per pulse (below).
 // kExact: 2 * halfwidth == W, so no tap lies past the half width.
 // `tab2` is the table in LDS or in global memory: each caller passes one of
 // the two, so that the reads compile to LDS or global loads.

@@ -142,7 +142,8 @@ def backproject(out, out_geometry: RadarGeometry, signal_data, in_geometry: Rada
 
     Extensions: ``precision`` "plain" (reference semantics, FP64 inner loop)
     or "split" (FP64 per-pixel reference + FP32 deltas), ``options`` tiling
-    dict {tile_rows, chunk, order, blocks_per_cu, staged, lane_rows}, ``stream`` (torch stream or raw hipStream_t int)
+    dict {tile_rows, chunk, order, blocks_per_cu, staged, lane_rows}, ``stream``
+    (torch stream or raw hipStream_t int),
     ``stats`` (dict filled with updates, geometry_ms, sum_ms, and for host
     pulses h2d_bytes, window_pulses, bands, copy_ms) and ``max_window_bytes``
     (device bytes for the pulse window of host pulses, 0 = half the free
