@@ -108,7 +108,7 @@ struct StaticData {
 
 // Per-pixel records, batch header + output descriptors, and the flags of one
 // call ([0] any failed, [1] out of range, [2] strips the line-interpolated sum
-// leaves, [8..9] update count, [16 + g] grid g failed).
+// leaves, [3] strips done again, [8..9] update count, [16 + g] grid g failed).
 struct Scratch {
     DevBuf geom, split, flags, desc;
     DevBuf strips, lines;   // line-interpolated sum: StripInfo, workspace
@@ -987,7 +987,7 @@ struct Step {
     bp::SumArgs sa;
     int width, precision;
     bool staged, pair;
-    int geom_grid, fit_grid, sum_grid;
+    int geom_grid, sum_grid;
     int32_t* flags;
     int flag_words;
     hipEvent_t ev[3];  // null: no timing
@@ -1180,7 +1180,6 @@ void build_step(Step& sp, const StaticData& st, const Scratch& sc, const CallArg
                                            : bp::sum_blocks_per_cu(a.precision, width, o.staged, sp.pair);
     sp.sum_grid = (n_cu * per_cu + 7) / 8 * 8;  // persistent split grid
     sp.geom_grid = 0;
-    sp.fit_grid = 0;
     sp.flags = d_flags;
     sp.flag_words = 0;
     sp.ev[0] = sp.ev[1] = sp.ev[2] = nullptr;
@@ -1197,7 +1196,7 @@ void set_lines(Step& sp, const LinePlan& p, const Scratch& sc, const CallArgs& a
     la.batch = sp.sa.batch;
     la.rec = reinterpret_cast<bp::PixLine*>(sc.split.ptr);
     la.info = static_cast<bp::StripInfo*>(sc.strips.ptr);
-    la.n_bad = sp.flags + 2;
+    la.n_left = sp.flags + 2;
     la.rc = sp.sa.rc;
     la.nr = gi.width;
     la.inv_k = sp.sa.inv_k;
@@ -1216,12 +1215,13 @@ void set_lines(Step& sp, const LinePlan& p, const Scratch& sc, const CallArgs& a
     sp.group_strips = group;
     sp.ga.strips = la.info;
     sp.sa.strips = la.info;
-    sp.sa.n_bad = la.n_bad;
+    sp.ga.strip_pass = sp.sa.strip_pass = bp::kPassLeft | bp::kPassRedo;
+    sp.sa.n_left = la.n_left;
 }
 
-// The coherent sum of a step over the descriptors at `batch`, reading pulse k
-// at rc + k * nr.
-int enqueue_sum(const Step& sp, const bp::BatchHeader* batch, const float2* rc, int plain_grid,
+// The coherent sum of a step over the descriptors at `batch` (`groups` groups of
+// four wavefront tiles), reading pulse k at rc + k * nr.
+int enqueue_sum(const Step& sp, const bp::BatchHeader* batch, const float2* rc, int groups,
                 int64_t n_strips, hipStream_t s)
 {
     bp::SumArgs sa = sp.sa;
@@ -1229,7 +1229,8 @@ int enqueue_sum(const Step& sp, const bp::BatchHeader* batch, const float2* rc, 
     sa.rc = rc;
     if (sp.lines) {
         // the strips in groups of the workspace's size, then the strips that
-        // did not qualify
+        // did not qualify or met samples that are not finite: their pixels'
+        // records are fitted only now
         bp::LineArgs la = sp.la;
         la.batch = batch;
         la.rc = rc;
@@ -1239,9 +1240,12 @@ int enqueue_sum(const Step& sp, const bp::BatchHeader* batch, const float2* rc, 
             la.s_end = s0 + n;
             BP_HIP_CHECK(bp::launch_strips(la, sp.width, true, s));
         }
+        bp::GeomArgs ga = sp.ga;
+        ga.batch = batch;
+        BP_HIP_CHECK(bp::launch_fit(ga, groups, s));
     }
     if (sp.precision == BP_PRECISION_PLAIN)
-        BP_HIP_CHECK(bp::launch_sum_plain(sa, sp.width, plain_grid, sp.segs, s));
+        BP_HIP_CHECK(bp::launch_sum_plain(sa, sp.width, groups, sp.segs, s));
     else
         BP_HIP_CHECK(bp::launch_sum_split(sa, sp.width, sp.sum_grid, sp.staged, sp.pair, s));
     return BP_SUCCESS;
@@ -1249,16 +1253,17 @@ int enqueue_sum(const Step& sp, const bp::BatchHeader* batch, const float2* rc, 
 
 // Enqueue the launches of one step: clear the flags, per-pixel geometry,
 // coherent sum (with optional event records around the two passes).
-int enqueue_step(const Step& sp, int plain_grid, hipStream_t s)
+int enqueue_step(const Step& sp, int groups, hipStream_t s)
 {
     BP_HIP_CHECK(bp::launch_clear(sp.flags, sp.flag_words, s));
     if (sp.ev[0]) BP_HIP_CHECK(hipEventRecord(sp.ev[0], s));
     BP_HIP_CHECK(bp::launch_geometry(sp.ga, sp.geom_grid, s));
     if (sp.lines)
         BP_HIP_CHECK(bp::launch_strip_fit(sp.ga, sp.la, bp::line_grid(bp::kLineFit, 0, sp.n_strips), s));
-    if (sp.precision == BP_PRECISION_SPLIT) BP_HIP_CHECK(bp::launch_fit(sp.ga, sp.fit_grid, s));
+    else if (sp.precision == BP_PRECISION_SPLIT)
+        BP_HIP_CHECK(bp::launch_fit(sp.ga, groups, s));
     if (sp.ev[1]) BP_HIP_CHECK(hipEventRecord(sp.ev[1], s));
-    const int rc = enqueue_sum(sp, sp.sa.batch, sp.sa.rc, plain_grid, sp.n_strips, s);
+    const int rc = enqueue_sum(sp, sp.sa.batch, sp.sa.rc, groups, sp.n_strips, s);
     if (rc != BP_SUCCESS) return rc;
     if (sp.ev[2]) BP_HIP_CHECK(hipEventRecord(sp.ev[2], s));
     return BP_SUCCESS;
@@ -1376,7 +1381,6 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
         sp.sa.parts_stride = n_rec;
     }
     sp.geom_grid = (int)hdr.n_geom_groups;
-    sp.fit_grid = (int)hdr.n_groups;
     sp.flag_words = 0;  // cleared above, before the pulse states
     if (stats)
         for (int i = 0; i < 3; ++i) sp.ev[i] = c->ev[i];
@@ -1623,7 +1627,6 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
     Step sp;
     build_step(sp, c->st, c->sc, a, width, o, c->n_cu);
     sp.geom_grid = (int)hdr.n_geom_groups;
-    sp.fit_grid = (int)hdr.n_groups;
     if (group > 0) set_lines(sp, lp, c->sc, a, hdr.n_strips, group);
 
     // geometry, the band windows (read back while the fit runs), the fit
@@ -1654,10 +1657,12 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
         if (hp.h_bad == nullptr)
             BP_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&hp.h_bad), sizeof(int32_t),
                                        hipHostMallocDefault));
-        BP_HIP_CHECK(hipMemcpyAsync(hp.h_bad, sp.la.n_bad, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        BP_HIP_CHECK(hipMemcpyAsync(hp.h_bad, sp.la.n_left, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     }
     BP_HIP_CHECK(hipEventRecord(hp.win_ev, s));
-    if (a.precision == BP_PRECISION_SPLIT) BP_HIP_CHECK(bp::launch_fit(sp.ga, sp.fit_grid, s));
+    // (with strips the fit follows them, in enqueue_sum)
+    if (a.precision == BP_PRECISION_SPLIT && !sp.lines)
+        BP_HIP_CHECK(bp::launch_fit(sp.ga, (int)hdr.n_groups, s));
     if (stats) BP_HIP_CHECK(hipEventRecord(c->ev[1], s));
     BP_HIP_CHECK(hipEventSynchronize(hp.win_ev));
 
@@ -1711,7 +1716,7 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
     };
     // pulses of a part: whole 64-pulse chunks
     const int64_t part = (int64_t)(budget / line_bytes) / 64 * 64;
-    bool any_part = false;
+    std::vector<std::pair<int64_t, int64_t>> part_rows;   // strip rows taken in parts
     if (sp.lines) {
         const int sr = whole.strip_rows;
         int64_t r = 0;
@@ -1728,7 +1733,7 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
                 sp.lines = false;
                 break;
             }
-            any_part = true;
+            part_rows.emplace_back(r, w.r1);
             for (int64_t q = w.k0 / 64 * 64; q < w.k1; q += part) {
                 Band b{r, w.r1, (int32_t)std::max<int64_t>(q, w.k0),
                        (int32_t)std::min<int64_t>(q + part, w.k1), Band::kPart};
@@ -1742,145 +1747,156 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
         if (!sp.lines) {
             // the pixel-by-pixel sum in bands of tile rows
             bands.clear();
-            any_part = false;
+            part_rows.clear();
             sp.ga.strips = nullptr;
             sp.sa.strips = nullptr;
-            BP_HIP_CHECK(bp::launch_fit(sp.ga, sp.fit_grid, s));
+            BP_HIP_CHECK(bp::launch_fit(sp.ga, (int)hdr.n_groups, s));
         }
     }
     if (!sp.lines) cut(0, length, band_rows, Band::kWhole);
-    if (any_part && (rc = ensure(hp.carry, bp::line_carry_bytes() * whole.strips_x))) return rc;
-    size_t max_band = 16;
-    for (const Band& b : bands)
-        if (b.k0 < b.k1) max_band = std::max(max_band, (size_t)(b.k1 - b.k0) * line_bytes);
-    const int nbuf = bands.size() > 1 && 2 * max_band <= budget ? 2 : 1;
-    for (int w = 0; w < nbuf; ++w)
-        if ((rc = ensure(hp.win[w], max_band))) return rc;
-    const int64_t chunk_lines = std::max<int64_t>(
-        1, std::min<int64_t>(batch, (int64_t)(kStageBytes / std::max<size_t>(line_bytes, 1))));
-    {
-        size_t have = hp.stage_bytes, have1 = hp.stage_bytes;
-        const size_t want = (size_t)chunk_lines * line_bytes;
-        if ((rc = ensure_pinned(hp.stage[0], have, want))) return rc;
-        if ((rc = ensure_pinned(hp.stage[1], have1, want))) return rc;
-        hp.stage_bytes = std::min(have, have1);
-    }
-
-    // descriptors of every band: the whole block's, cut to the band's lines
-    const size_t stride = (sizeof(bp::BatchHeader) + sizeof(bp::OutDesc) + 255) & ~size_t(255);
-    std::vector<unsigned char> bdesc(stride * bands.size(), 0);
-    std::vector<int> band_groups(bands.size());
-    std::vector<int64_t> band_strips(bands.size());
-    for (size_t b = 0; b < bands.size(); ++b) {
-        bp::OutDesc d = whole;
-        const int64_t r0 = bands[b].r0;
-        d.map = make_map(bands[b].r1 - r0, owidth, o.tile_rows, o.order, o.lane_rows);
-        d.t0 = whole.t0 + r0 * whole.dt;
-        d.seq_base = 0;
-        d.rec_base = whole.rec_base + r0 * owidth;
-        d.out = whole.out + r0 * owidth;
-        d.height = whole.height ? whole.height + r0 * owidth : nullptr;
-        d.strip_seq = 0;
-        d.strip_info = whole.strip_info + r0 / whole.strip_rows * whole.strips_x;
-        d.strips_y = (int32_t)((d.map.length + d.strip_rows - 1) / d.strip_rows);
-        bp::BatchHeader h;
-        std::memset(&h, 0, sizeof(h));
-        h.n_seq = d.map.n_tiles;
-        h.n_groups = (h.n_seq + 3) / 4;
-        h.n_geom_groups = (h.n_seq * o.lane_rows + 3) / 4;
-        h.n_grids = 1;
-        h.lane_rows = o.lane_rows;
-        h.n_strips = (int64_t)d.strips_x * d.strips_y;
-        std::memcpy(bdesc.data() + b * stride, &h, sizeof(h));
-        std::memcpy(bdesc.data() + b * stride + sizeof(h), &d, sizeof(d));
-        band_groups[b] = (int)h.n_groups;
-        band_strips[b] = h.n_strips;
-    }
-    if ((rc = upload(hp.band_desc, bdesc.data(), bdesc.size(), s))) return rc;
-
+    if (!part_rows.empty() && (rc = ensure(hp.carry, bp::line_carry_bytes() * whole.strips_x))) return rc;
     const bool timed = stats != nullptr || hstats != nullptr;
-    while (timed && hp.timing.size() < 4 * bands.size()) {
-        hipEvent_t e;
-        BP_HIP_CHECK(hipEventCreate(&e));
-        hp.timing.push_back(e);
-    }
-    // copies on the copy stream (they write only the context's window
-    // buffers, which no earlier call still reads: every call ends with both
-    // streams drained), sums on the caller's stream
-    const unsigned char* src = static_cast<const unsigned char*>(a.in_dev);
-    int64_t h2d = 0, pulses = 0, chunk_no = 0;
-    bool used[2] = {false, false};
-    for (size_t b = 0; b < bands.size(); ++b) {
-        const Band& bd = bands[b];
-        const int w = (int)(b % nbuf);
-        unsigned char* dwin = static_cast<unsigned char*>(hp.win[w].ptr);
-        if (used[w]) BP_HIP_CHECK(hipStreamWaitEvent(hp.copy, hp.sum_ev[w], 0));
-        if (timed) BP_HIP_CHECK(hipEventRecord(hp.timing[4 * b], hp.copy));
-        for (int64_t k = bd.k0; k < bd.k1; k += chunk_lines) {
-            const int64_t n = std::min<int64_t>(chunk_lines, bd.k1 - k);
-            const int j = (int)(chunk_no++ & 1);
-            // staging j is free once its previous copy has finished
-            BP_HIP_CHECK(hipEventSynchronize(hp.stage_ev[j]));
-            const size_t bytes = (size_t)n * line_bytes;
-            host_copy(hp.stage[j], src + (size_t)k * line_bytes, bytes);
-            BP_HIP_CHECK(hipMemcpyAsync(dwin + (size_t)(k - bd.k0) * line_bytes, hp.stage[j],
-                                        bytes, hipMemcpyHostToDevice, hp.copy));
-            BP_HIP_CHECK(hipEventRecord(hp.stage_ev[j], hp.copy));
-            h2d += (int64_t)bytes;
-        }
-        if (bd.k0 < bd.k1) pulses += bd.k1 - bd.k0;
-        if (timed) BP_HIP_CHECK(hipEventRecord(hp.timing[4 * b + 1], hp.copy));
-        BP_HIP_CHECK(hipEventRecord(hp.copied_ev, hp.copy));
-        BP_HIP_CHECK(hipStreamWaitEvent(s, hp.copied_ev, 0));
-        // pulse k of the band at dwin + (k - k0) * line_bytes; the sum reads
-        // only pulses of its pixels' windows, all inside [k0, k1)
-        const int64_t k0 = bd.k0 < bd.k1 ? bd.k0 : 0;
-        const float2* rc_base = reinterpret_cast<const float2*>(
-            reinterpret_cast<uintptr_t>(dwin) - (uintptr_t)((size_t)k0 * line_bytes));
-        const auto* batch_b = reinterpret_cast<const bp::BatchHeader*>(
-            static_cast<unsigned char*>(hp.band_desc.ptr) + b * stride);
-        if (timed) BP_HIP_CHECK(hipEventRecord(hp.timing[4 * b + 2], s));
-        if (bd.kind == Band::kPart) {
-            bp::LineArgs la = sp.la;
-            la.batch = batch_b;
-            la.rc = rc_base;
-            la.s_begin = 0;
-            la.s_end = band_strips[b];
-            la.q_begin = bd.k0 / 64 * 64;
-            la.q_end = bd.k1;
-            la.q_first = bd.first;
-            la.carry = static_cast<double2*>(hp.carry.ptr);
-            BP_HIP_CHECK(bp::launch_strips(la, sp.width, bd.last, s));
-        } else if ((rc = enqueue_sum(sp, batch_b, rc_base, band_groups[b],
-                                     bd.kind == Band::kTiles ? 0 : band_strips[b], s))) {
-            return rc;
-        }
-        if (timed) BP_HIP_CHECK(hipEventRecord(hp.timing[4 * b + 3], s));
-        BP_HIP_CHECK(hipEventRecord(hp.sum_ev[w], s));
-        used[w] = true;
-    }
-    if (stats) BP_HIP_CHECK(hipEventRecord(c->ev[2], s));
-
-    c->flags_host.assign(n_flag, 0);
-    BP_HIP_CHECK(hipMemcpyAsync(c->flags_host.data(), c->sc.flags.ptr, sizeof(int32_t) * n_flag,
-                                hipMemcpyDeviceToHost, s));
-    BP_HIP_CHECK(hipStreamSynchronize(s));
-    BP_HIP_CHECK(hipStreamSynchronize(hp.copy));
-    drain.armed = false;
+    int64_t h2d = 0, pulses = 0;
+    size_t n_bands = 0;
     double sum_ms = 0., copy_ms = 0.;
-    if (timed) {
-        for (size_t b = 0; b < bands.size(); ++b) {
-            float ms = 0.f;
-            BP_HIP_CHECK(hipEventElapsedTime(&ms, hp.timing[4 * b], hp.timing[4 * b + 1]));
-            copy_ms += ms;
-            BP_HIP_CHECK(hipEventElapsedTime(&ms, hp.timing[4 * b + 2], hp.timing[4 * b + 3]));
-            sum_ms += ms;
+    for (bool again = false;; again = true) {
+        drain.armed = true;
+        size_t max_band = 16;
+        for (const Band& b : bands)
+            if (b.k0 < b.k1) max_band = std::max(max_band, (size_t)(b.k1 - b.k0) * line_bytes);
+        const int nbuf = bands.size() > 1 && 2 * max_band <= budget ? 2 : 1;
+        for (int w = 0; w < nbuf; ++w)
+            if ((rc = ensure(hp.win[w], max_band))) return rc;
+        const int64_t chunk_lines = std::max<int64_t>(
+            1, std::min<int64_t>(batch, (int64_t)(kStageBytes / std::max<size_t>(line_bytes, 1))));
+        {
+            size_t have = hp.stage_bytes, have1 = hp.stage_bytes;
+            const size_t want = (size_t)chunk_lines * line_bytes;
+            if ((rc = ensure_pinned(hp.stage[0], have, want))) return rc;
+            if ((rc = ensure_pinned(hp.stage[1], have1, want))) return rc;
+            hp.stage_bytes = std::min(have, have1);
         }
+
+        // descriptors of every band: the whole block's, cut to the band's lines
+        const size_t stride = (sizeof(bp::BatchHeader) + sizeof(bp::OutDesc) + 255) & ~size_t(255);
+        std::vector<unsigned char> bdesc(stride * bands.size(), 0);
+        std::vector<int> band_groups(bands.size());
+        std::vector<int64_t> band_strips(bands.size());
+        for (size_t b = 0; b < bands.size(); ++b) {
+            bp::OutDesc d = whole;
+            const int64_t r0 = bands[b].r0;
+            d.map = make_map(bands[b].r1 - r0, owidth, o.tile_rows, o.order, o.lane_rows);
+            d.t0 = whole.t0 + r0 * whole.dt;
+            d.seq_base = 0;
+            d.rec_base = whole.rec_base + r0 * owidth;
+            d.out = whole.out + r0 * owidth;
+            d.height = whole.height ? whole.height + r0 * owidth : nullptr;
+            d.strip_seq = 0;
+            d.strip_info = whole.strip_info + r0 / whole.strip_rows * whole.strips_x;
+            d.strips_y = (int32_t)((d.map.length + d.strip_rows - 1) / d.strip_rows);
+            bp::BatchHeader h;
+            std::memset(&h, 0, sizeof(h));
+            h.n_seq = d.map.n_tiles;
+            h.n_groups = (h.n_seq + 3) / 4;
+            h.n_geom_groups = (h.n_seq * o.lane_rows + 3) / 4;
+            h.n_grids = 1;
+            h.lane_rows = o.lane_rows;
+            h.n_strips = (int64_t)d.strips_x * d.strips_y;
+            std::memcpy(bdesc.data() + b * stride, &h, sizeof(h));
+            std::memcpy(bdesc.data() + b * stride + sizeof(h), &d, sizeof(d));
+            band_groups[b] = (int)h.n_groups;
+            band_strips[b] = h.n_strips;
+        }
+        if ((rc = upload(hp.band_desc, bdesc.data(), bdesc.size(), s))) return rc;
+
+        while (timed && hp.timing.size() < 4 * bands.size()) {
+            hipEvent_t e;
+            BP_HIP_CHECK(hipEventCreate(&e));
+            hp.timing.push_back(e);
+        }
+        // copies on the copy stream (they write only the context's window
+        // buffers, which no earlier call still reads: every call ends with both
+        // streams drained), sums on the caller's stream
+        const unsigned char* src = static_cast<const unsigned char*>(a.in_dev);
+        int64_t chunk_no = 0;
+        bool used[2] = {false, false};
+        for (size_t b = 0; b < bands.size(); ++b) {
+            const Band& bd = bands[b];
+            const int w = (int)(b % nbuf);
+            unsigned char* dwin = static_cast<unsigned char*>(hp.win[w].ptr);
+            if (used[w]) BP_HIP_CHECK(hipStreamWaitEvent(hp.copy, hp.sum_ev[w], 0));
+            if (timed) BP_HIP_CHECK(hipEventRecord(hp.timing[4 * b], hp.copy));
+            for (int64_t k = bd.k0; k < bd.k1; k += chunk_lines) {
+                const int64_t n = std::min<int64_t>(chunk_lines, bd.k1 - k);
+                const int j = (int)(chunk_no++ & 1);
+                // staging j is free once its previous copy has finished
+                BP_HIP_CHECK(hipEventSynchronize(hp.stage_ev[j]));
+                const size_t bytes = (size_t)n * line_bytes;
+                host_copy(hp.stage[j], src + (size_t)k * line_bytes, bytes);
+                BP_HIP_CHECK(hipMemcpyAsync(dwin + (size_t)(k - bd.k0) * line_bytes, hp.stage[j],
+                                            bytes, hipMemcpyHostToDevice, hp.copy));
+                BP_HIP_CHECK(hipEventRecord(hp.stage_ev[j], hp.copy));
+                h2d += (int64_t)bytes;
+            }
+            if (bd.k0 < bd.k1) pulses += bd.k1 - bd.k0;
+            if (timed) BP_HIP_CHECK(hipEventRecord(hp.timing[4 * b + 1], hp.copy));
+            BP_HIP_CHECK(hipEventRecord(hp.copied_ev, hp.copy));
+            BP_HIP_CHECK(hipStreamWaitEvent(s, hp.copied_ev, 0));
+            // pulse k of the band at dwin + (k - k0) * line_bytes; the sum reads
+            // only pulses of its pixels' windows, all inside [k0, k1)
+            const int64_t k0 = bd.k0 < bd.k1 ? bd.k0 : 0;
+            const float2* rc_base = reinterpret_cast<const float2*>(
+                reinterpret_cast<uintptr_t>(dwin) - (uintptr_t)((size_t)k0 * line_bytes));
+            const auto* batch_b = reinterpret_cast<const bp::BatchHeader*>(
+                static_cast<unsigned char*>(hp.band_desc.ptr) + b * stride);
+            if (timed) BP_HIP_CHECK(hipEventRecord(hp.timing[4 * b + 2], s));
+            if (bd.kind == Band::kPart) {
+                bp::LineArgs la = sp.la;
+                la.batch = batch_b;
+                la.rc = rc_base;
+                la.s_begin = 0;
+                la.s_end = band_strips[b];
+                la.q_begin = bd.k0 / 64 * 64;
+                la.q_end = bd.k1;
+                la.q_first = bd.first;
+                la.carry = static_cast<double2*>(hp.carry.ptr);
+                BP_HIP_CHECK(bp::launch_strips(la, sp.width, bd.last, s));
+            } else if ((rc = enqueue_sum(sp, batch_b, rc_base, band_groups[b],
+                                         bd.kind == Band::kTiles ? 0 : band_strips[b], s))) {
+                return rc;
+            }
+            if (timed) BP_HIP_CHECK(hipEventRecord(hp.timing[4 * b + 3], s));
+            BP_HIP_CHECK(hipEventRecord(hp.sum_ev[w], s));
+            used[w] = true;
+        }
+        if (stats) BP_HIP_CHECK(hipEventRecord(c->ev[2], s));
+
+        c->flags_host.assign(n_flag, 0);
+        BP_HIP_CHECK(hipMemcpyAsync(c->flags_host.data(), c->sc.flags.ptr, sizeof(int32_t) * n_flag,
+                                    hipMemcpyDeviceToHost, s));
+        BP_HIP_CHECK(hipStreamSynchronize(s));
+        BP_HIP_CHECK(hipStreamSynchronize(hp.copy));
+        drain.armed = false;
+        n_bands += bands.size();
+        if (timed) {
+            for (size_t b = 0; b < bands.size(); ++b) {
+                float ms = 0.f;
+                BP_HIP_CHECK(hipEventElapsedTime(&ms, hp.timing[4 * b], hp.timing[4 * b + 1]));
+                copy_ms += ms;
+                BP_HIP_CHECK(hipEventElapsedTime(&ms, hp.timing[4 * b + 2], hp.timing[4 * b + 3]));
+                sum_ms += ms;
+            }
+        }
+        // strips taken in parts met samples that are not finite, and no bands of
+        // tile rows followed them: those rows once more, pixel by pixel
+        if (again || part_rows.empty() || *hp.h_bad > 0 || c->flags_host[3] == 0) break;
+        bands.clear();
+        for (const auto& r : part_rows) cut(r.first, r.second, band_rows, Band::kTiles);
     }
     if (hstats) {
         hstats->h2d_bytes = h2d;
         hstats->window_pulses = pulses;
-        hstats->bands = (int32_t)bands.size();
+        hstats->bands = (int32_t)n_bands;
         hstats->copy_ms = copy_ms;
     }
     const hipEvent_t ev[3] = {stats ? c->ev[0] : nullptr, nullptr, stats ? c->ev[2] : nullptr};
@@ -2030,7 +2046,6 @@ int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
     // group counts (bp_scene_focus); one workgroup at capture
     const int cap_grid = 1;
     sp.geom_grid = cap_grid;
-    sp.fit_grid = cap_grid;
     sp.flag_words = kFlagWords + sc->max_blocks;
     // no event records inside the graph: a replay is timed as a whole by
     // events recorded around the launch

@@ -204,11 +204,18 @@ constexpr float kLinePosTol = 1e-4f, kLinePosMax = 3e-3f;
 constexpr int kSlopeNodes = 4;
 constexpr float kLineColumnTol = 0.06f;  // bins: fractional positions of the columns
 
+// What becomes of a strip: left to the pixel-by-pixel sum by its fit, taken by
+// the line-interpolated sum, or taken and, with sums that are not finite, done
+// again by the pixel-by-pixel sum.
+enum StripState : int32_t { kStripLeft = 0, kStripTaken = 1, kStripRedo = 2 };
+// The strips that a launch of the pixel-by-pixel sum (and of its fit) takes.
+enum StripPass : int32_t { kPassLeft = 1, kPassRedo = 2 };
+
 // Pulses of a strip: k0 .. k1 by some pixel, f0 .. f1 by all; chunks of
 // 2^chunk_log2 pulses (absolute multiples) from slot0.
 struct StripInfo {
     int32_t k0, k1, f0, f1;
-    int32_t ok;
+    int32_t ok;              // StripState
     int32_t slot0, nslots;
     int32_t slopes;          // the lines' positions need the samples' derivatives
 };
@@ -230,7 +237,7 @@ struct LineArgs {
     const BatchHeader* batch;
     PixLine* rec;
     StripInfo* info;
-    int32_t* n_bad;                      // strips left to the pixel-by-pixel sum
+    int32_t* n_left;                     // strips left to the pixel-by-pixel sum, and done again
     const float2* rc;                    // range-compressed pulses [na x nr]
     int64_t nr;
     double inv_k;                        // 1 / (fc dtau): cycles -> range bins
@@ -277,9 +284,10 @@ struct GeomArgs {
     PixGeom* geom;              // plain records (always written)
     PixSplit* split;            // split records (when want_split)
     int32_t* flags;             // [0] any failed, [1] out of range, [2] strips
-                                // left to the pixel-by-pixel split sum
+                                // left to the pixel-by-pixel split sum, [3] done again
     unsigned long long* updates;
     const StripInfo* strips;    // line-interpolated sum's strips, or null
+    int32_t strip_pass;         // StripPass bits of this launch
 };
 
 struct SumArgs {
@@ -304,8 +312,9 @@ struct SumArgs {
     double inv_dtau;            // 1 / dtau
     const double2* tab2;        // plain: (t_i, t_{i+1} - t_i) per table entry, as doubles
     double fold_c[4];           // split: n, C(n,2), C(n,3), C(n,4) for n = chunk
-    const StripInfo* strips;    // split: strips summed by line interpolation, or null
-    const int32_t* n_bad;       // strips that are not
+    const StripInfo* strips;    // split: strips of the line-interpolated sum, or null
+    const int32_t* n_left;      // strips left, and done again
+    int32_t strip_pass;         // StripPass bits of this launch
     double2* parts;             // plain: segment sums [segment][record], or null
     int64_t parts_stride;       // records per segment
 };

@@ -268,15 +268,24 @@ __device__ inline PixSplit fit_pixel(const GeomArgs& a, const PixGeom& g, bool h
     return sp;
 }
 
-// Whether wavefront tile `tile` of grid d lies in a strip that the
-// line-interpolated sum takes (a tile never straddles strips: strip heights
-// are multiples of 16, its widths of 64).
-__device__ inline bool strip_done(const StripInfo* strips, const OutDesc& d, int64_t tile)
+// Whether wavefront tile `tile` of grid d lies in a strip that a launch with
+// these StripPass bits passes over (a tile never straddles strips: strip
+// heights are multiples of 16, its widths of 64).
+__device__ inline bool strip_skipped(const StripInfo* strips, int pass, const OutDesc& d,
+                                     int64_t tile)
 {
     const int64_t ty = tile / d.map.tiles_x, tx = tile - ty * d.map.tiles_x;
     const int64_t y = ty * d.map.tile_rows * d.map.lane_rows / d.strip_rows;
     const int64_t x = tx * d.map.tile_cols / 64;
-    return __builtin_amdgcn_readfirstlane(strips[d.strip_info + y * d.strips_x + x].ok) != 0;
+    const int ok = __builtin_amdgcn_readfirstlane(strips[d.strip_info + y * d.strips_x + x].ok);
+    return !((ok == kStripLeft && (pass & kPassLeft)) || (ok == kStripRedo && (pass & kPassRedo)));
+}
+
+// Whether such a launch has no strip at all.
+__device__ inline bool pass_empty(const int32_t* n_left, int pass)
+{
+    const int n = ((pass & kPassLeft) ? n_left[0] : 0) + ((pass & kPassRedo) ? n_left[1] : 0);
+    return __builtin_amdgcn_readfirstlane(n) == 0;
 }
 
 // One sum wavefront tile: read the geometry records of its pixels (lane_rows
@@ -286,7 +295,8 @@ __device__ inline void fit_tile(const GeomArgs& a, const OutDesc* grids, int n_g
 {
     const bool in_seq = gseq < n_seq;
     const OutDesc d = load_desc(grids, in_seq ? find_grid(grids, n_grids, gseq) : 0);
-    if (a.strips != nullptr && in_seq && strip_done(a.strips, d, gseq - d.seq_base)) return;
+    if (a.strips != nullptr && in_seq && strip_skipped(a.strips, a.strip_pass, d, gseq - d.seq_base))
+        return;
     const int lr = d.map.lane_rows;  // 1 or 2
     bool valid[2] = {false, false}, has_win[2] = {false, false};
     int64_t rec[2] = {0, 0};
@@ -358,7 +368,7 @@ void fit_kernel(GeomArgs a)
 {
     const int64_t ng = uniform64(a.batch->n_groups);
     if ((int64_t)blockIdx.x >= ng) return;
-    if (a.strips != nullptr && __builtin_amdgcn_readfirstlane(a.flags[2]) == 0) return;
+    if (a.strips != nullptr && pass_empty(a.flags + 2, a.strip_pass)) return;
     const OutDesc* grids = batch_grids(a.batch);
     const int n_grids = __builtin_amdgcn_readfirstlane(a.batch->n_grids);
     const int64_t n_seq = uniform64(a.batch->n_seq);
@@ -1444,7 +1454,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 void sum_split_kernel(SumArgs a)
 {
     static_assert(!(kPair && kStaged), "two-line lanes gather their taps");
-    if (a.strips != nullptr && __builtin_amdgcn_readfirstlane(*a.n_bad) == 0) return;
+    if (a.strips != nullptr && pass_empty(a.n_left, a.strip_pass)) return;
     constexpr int ROW = poly_row_floats(W);
     constexpr int kTable = kPair ? PairTable<W>::kFloats : (kPolyphaseRows + 1) * ROW;
     // static LDS arrays: row and slot offsets fold into the ds_read offsets
@@ -1456,7 +1466,9 @@ void sum_split_kernel(SumArgs a)
     __syncthreads();
     char* s_win = reinterpret_cast<char*>(s_win4);
     for_each_tile(a.batch, [&](const OutDesc& d, int64_t tile, int lane) {
-        if (a.strips != nullptr && tile < d.map.n_tiles && strip_done(a.strips, d, tile)) return;
+        if (a.strips != nullptr && tile < d.map.n_tiles &&
+            strip_skipped(a.strips, a.strip_pass, d, tile))
+            return;
         if constexpr (kPair)
             pair_tile<W>(a, s_poly, d, tile, lane);
         else

@@ -14,7 +14,8 @@
 //                centre, an FP64 sum; and the corrections of the next paragraph
 //   strip_ends   the pulses at the ends of the aperture that only some of the
 //                strip's lines integrate, line by line
-//   strip_sum    the partial sums of a pixel, added in a fixed order
+//   strip_sum    the partial sums of a pixel, added in a fixed order; strips
+//                where one is not finite are left to the pixel-by-pixel sum
 //
 // The interpolated pulse sample s(u) is only piecewise smooth in the range
 // position u: where u enters the next bin, a tap of the (truncated) kernel
@@ -52,6 +53,8 @@
 // bp_internal.h, the nodes reproduce every line's phase slope, and the
 // columns' fractional bins agree (corrections would otherwise be needed at
 // most pulses); the others take the pixel-by-pixel sum.
+#include <float.h>
+
 #include "bp_device.h"
 
 namespace bp {
@@ -321,8 +324,8 @@ void strip_fit_kernel(GeomArgs a, LineArgs l)
     const int nslots = ((f1 - 1) >> l.chunk_log2) - slot0 + 1;
     if (!__builtin_amdgcn_readfirstlane(ok) || f0 >= f1 || nslots > l.slots) {
         if (threadIdx.x == 0) {
-            l.info[st.info] = StripInfo{k0, k1, f0, f1, 0, 0, 0, 0};
-            atomicAdd(l.n_bad, 1);
+            l.info[st.info] = StripInfo{k0, k1, f0, f1, kStripLeft, 0, 0, 0};
+            atomicAdd(l.n_left, 1);
         }
         return;
     }
@@ -432,9 +435,9 @@ void strip_fit_kernel(GeomArgs a, LineArgs l)
     if (slopes) s_slopes = 1;
     __syncthreads();
     if (threadIdx.x == 0) {
-        const int good = s_bad == 0;
-        l.info[st.info] = StripInfo{k0, k1, f0, f1, good, slot0, nslots, s_slopes};
-        if (!good) atomicAdd(l.n_bad, 1);
+        const int ok = s_bad == 0 ? kStripTaken : kStripLeft;
+        l.info[st.info] = StripInfo{k0, k1, f0, f1, ok, slot0, nslots, s_slopes};
+        if (ok == kStripLeft) atomicAdd(l.n_left, 1);
     }
 }
 
@@ -1007,7 +1010,11 @@ void strip_ends_kernel(LineArgs a)
     group_sums<W, true>(a);
 }
 
-// The partial sums of each pixel of a strip, in segment order.
+// The partial sums of each pixel of a strip, in segment order.  A strip with a
+// sum that is not finite is left to the pixel-by-pixel sum: a NaN or an
+// infinity among the pulses reaches every line of a column through the node
+// sums and the corrections (never none of those that integrate it), and pixels
+// whose own taps miss it keep their finite values there.
 __global__ __launch_bounds__(kLineThreads) void strip_sum_kernel(LineArgs a)
 {
     constexpr int kPer = kStripLines * 64 / kLineThreads / 4;   // pixels per thread
@@ -1021,6 +1028,7 @@ __global__ __launch_bounds__(kLineThreads) void strip_sum_kernel(LineArgs a)
     const Strip st = load_strip(d, t);
     if (!(uniform_ptr(a.info) + st.info)->ok) return;
     const float2* e = a.parts + ws * kSegs * (kStripLines * 64);
+    bool bad = false;
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
         const int i = ((int)(blockIdx.x & 3) * kPer + q) * (kLineThreads / 64) + (threadIdx.x >> 6);
@@ -1033,8 +1041,13 @@ __global__ __launch_bounds__(kLineThreads) void strip_sum_kernel(LineArgs a)
             re += (double)v.x;
             im += (double)v.y;
         }
-        st.out[st.pix0 + i * st.width + lane] = make_float2((float)re, (float)im);
+        const float2 z = make_float2((float)re, (float)im);
+        bad |= !(fabsf(z.x) <= FLT_MAX && fabsf(z.y) <= FLT_MAX);
+        st.out[st.pix0 + i * st.width + lane] = z;
     }
+    if (__syncthreads_or(bad) && threadIdx.x == 0 &&
+        atomicExch(&a.info[st.info].ok, kStripRedo) != kStripRedo)
+        atomicAdd(a.n_left + 1, 1);
 }
 
 }  // namespace
