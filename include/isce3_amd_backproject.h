@@ -232,7 +232,8 @@ int bp_backproject(bp_context* ctx, const bp_radar_geometry* out_geometry,
  * address is looked up by bp_context_create.  A call whose buffers do not fit
  * (the records take bp_scratch_bytes_per_pixel(precision) bytes per output
  * pixel: 48 plain, 112 split, so about 2.7 M plain or 1.1 M split pixels with
- * small tables) fails with BP_ERR_LENGTH before any launch.  The call makes
+ * small tables) fails with BP_ERR_LENGTH before any launch.  32 MiB more of the
+ * array are kept for the sums' workspace.  The call makes
  * no hipMalloc, hipFree, pinned or library allocation on the device; its
  * table uploads are pageable host-to-device copies on `stream`.
  *

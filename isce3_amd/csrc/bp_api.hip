@@ -592,8 +592,12 @@ void build_plain_table(const bp_kernel& k, std::vector<double>& out)
 // passes `scratch` itself (in host code the name is a stand-in, not a device
 // address): bp_context_create looks up each device's address once, with that
 // device current, and every use goes through that address.
+// Behind the part that limits what a call may hold lies room for the strips of
+// the line-interpolated sum, so that which sum a pixel takes does not depend on
+// how full the first part is.
 constexpr size_t kNoAllocScratchBytes = size_t(BP_NOALLOC_SCRATCH_MIB) << 20;
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+constexpr size_t kNoAllocLineBytes = size_t(32) << 20;
+static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes + kNoAllocLineBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -724,6 +728,9 @@ namespace {
 
 // Workspace of the line-interpolated sum at most; more strips run in groups.
 constexpr size_t kLineBytes = size_t(1536) << 20;
+// ... and that of one strip (300,000 pulses of aperture), for which every call
+// has room.
+constexpr size_t kStripBytes = size_t(24) << 20;
 constexpr int kFlagWords = 16;  // flag words in front of the per-grid flags
 
 // Arguments shared by every output block of a call (the raw set and its
@@ -1051,7 +1058,7 @@ LinePlan plan_lines(const CallArgs& a, int width, const Opts& o)
     p.table.tropo = a.tropo;
     p.table.n_sums = 8 + (a.tropo != BP_TROPO_NODELAY ? bp::kSlopeNodes : 0);
     p.strip_bytes = bp::line_strip_bytes(p.slots, p.table.n_sums);
-    p.on = p.strip_bytes <= kLineBytes;
+    p.on = p.strip_bytes <= kStripBytes;
     return p;
 }
 
@@ -1362,8 +1369,6 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
     int64_t group = 0;
     if (lp.on) {
         if (carve) {
-            // what the call's own buffers leave of the fixed scratch, if it
-            // holds a strip
             group = carve_lines(*carve, lp, hdr.n_strips, sc);
         } else {
             group = alloc_lines(lp, hdr.n_strips, sc);
@@ -1466,7 +1471,8 @@ int carve_call(Carve& cv, const CallArgs& a, int width, int n_blocks, int64_t np
     return BP_SUCCESS;
 }
 
-// Segment sums of the plain sum in what a no-alloc call's buffers leave.
+// Segment sums of the plain sum in what a no-alloc call's buffers leave (the
+// sums are the same without them).
 int carve_parts(Carve& cv, size_t bytes, Scratch& sc)
 {
     if (cv.used > cv.cap || bytes + 256 > cv.cap - cv.used) return BP_ERR_LENGTH;
@@ -1474,10 +1480,15 @@ int carve_parts(Carve& cv, size_t bytes, Scratch& sc)
 }
 
 // Workspace of the line-interpolated sum in what a no-alloc call's buffers
-// leave; the strips it holds (0: none, the call sums pixel by pixel).
+// leave and the room kept for it, which holds a strip of any call and the
+// StripInfo of all that its records allow (16 lines of one pixel each).
 int64_t carve_lines(Carve& cv, const LinePlan& p, int64_t n_strips, Scratch& sc)
 {
     const size_t info = sizeof(bp::StripInfo) * (size_t)n_strips;
+    static_assert(kStripBytes + sizeof(bp::StripInfo) * (kNoAllocScratchBytes /
+                  (sizeof(bp::PixGeom) + sizeof(bp::PixSplit)) / 16 + 1) + 1024 <= kNoAllocLineBytes,
+                  "room for a strip");
+    cv.cap = kNoAllocScratchBytes + kNoAllocLineBytes;
     if (cv.used > cv.cap || info + p.strip_bytes + 512 > cv.cap - cv.used) return 0;
     const int64_t group =
         std::min<int64_t>(n_strips, (int64_t)((cv.cap - cv.used - info - 512) / p.strip_bytes));

@@ -109,6 +109,27 @@ def test_no_device_memory_taken(torch_gpu, raws):
         _native.lib().bp_context_destroy(h)
 
 
+def test_same_results_at_the_limit(torch_gpu, ctx):
+    """The largest split call that fits: its strips have the room kept for them,
+    in several groups, and the results are bp_backproject's."""
+    from isce3_amd import _native, sim
+    sc = sim.make_scene("tiny")
+    na, nr = 700, 1200
+    sc.in_grid = sim._grid(-0.5 * na / sim.PRF, sim.PRF, sim.R0, sim.DR, na, nr)
+    gen = torch_gpu.Generator(device="cuda:0")
+    gen.manual_seed(3)
+    d_raw = torch_gpu.randn((na, nr), dtype=torch_gpu.complex64, device="cuda:0", generator=gen)
+    for rows in range(1097, 1000, -1):
+        g = sim._grid(-0.5 * rows / sim.PRF, sim.PRF, sim.R0 + 40 * sim.DR, sim.DR, rows, 1092)
+        got = _call("bp_backproject_noalloc", ctx, torch_gpu, sc, d_raw, g, "split")
+        if got[0] != _native.BP_ERR_LENGTH:
+            break
+    assert got[0] == 0 and 1060 <= rows < 1097
+    want = _call("bp_backproject", ctx, torch_gpu, sc, d_raw, g, "split")
+    np.testing.assert_array_equal(got[1], want[1])
+    np.testing.assert_array_equal(got[2], want[2])
+
+
 def test_oversized_call_refused_then_next_call_works(torch_gpu, ctx, raws):
     from isce3_amd import _native
     from isce3_amd.product import RadarGridParameters
