@@ -1215,7 +1215,7 @@ void set_lines(Step& sp, const LinePlan& p, const Scratch& sc, const CallArgs& a
     la.s_end = group;
     la.q_begin = INT32_MIN;
     la.q_end = INT32_MAX;
-    la.few = n <= bp::kFewStrips ? 1 : 0;
+    la.few = std::min(n, group) <= bp::kFewStrips ? 1 : 0;
     bp::line_place(la, static_cast<unsigned char*>(sc.lines.ptr), group);
     sp.lines = true;
     sp.n_strips = n;
