@@ -275,7 +275,9 @@ typedef struct {
  * read.  When that window exceeds max_window_bytes of device memory, the
  * block is focused in bands of output lines, each with its own window.  The
  * results equal bp_backproject's with the whole raster on the device, bit for
- * bit, in every case.
+ * bit, in every case (short of a device without room for the half megabyte that
+ * one strip of the line-interpolated split sum takes: there either call sums
+ * pixel by pixel, 1e-4 relative).
  *
  *   in_host            host, complex64 [in.grid.length x in.grid.width]
  *   batch              pulses per host-to-device copy (>= 1, else BP_ERR_DOMAIN)

@@ -1087,8 +1087,9 @@ int64_t line_group(const LinePlan& p, int64_t n)
     return std::min<int64_t>(n, (int64_t)(kLineBytes / p.strip_bytes));
 }
 
-// Workspace for n strips, as many at once as the device has room for (their
-// number; 0: not even one, the call sums pixel by pixel).
+// Workspace for n strips, as many at once as the device has room for: their
+// number.  Results do not depend on it, but for a device without room for a
+// single strip (0.3 to 0.5 MB), where the call sums pixel by pixel (0).
 int64_t alloc_lines(const LinePlan& p, int64_t n, Scratch& sc)
 {
     if (ensure(sc.strips, sizeof(bp::StripInfo) * n) != BP_SUCCESS) return 0;
@@ -1484,11 +1485,11 @@ int carve_parts(Carve& cv, size_t bytes, Scratch& sc)
 // StripInfo of all that its records allow (16 lines of one pixel each).
 int64_t carve_lines(Carve& cv, const LinePlan& p, int64_t n_strips, Scratch& sc)
 {
-    const size_t info = sizeof(bp::StripInfo) * (size_t)n_strips;
     static_assert(kStripBytes + sizeof(bp::StripInfo) * (kNoAllocScratchBytes /
                   (sizeof(bp::PixGeom) + sizeof(bp::PixSplit)) / 16 + 1) + 1024 <= kNoAllocLineBytes,
                   "room for a strip");
     cv.cap = kNoAllocScratchBytes + kNoAllocLineBytes;
+    const size_t info = sizeof(bp::StripInfo) * (size_t)n_strips;
     if (cv.used > cv.cap || info + p.strip_bytes + 512 > cv.cap - cv.used) return 0;
     const int64_t group =
         std::min<int64_t>(n_strips, (int64_t)((cv.cap - cv.used - info - 512) / p.strip_bytes));
@@ -1740,7 +1741,8 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
             // a strip row whose window is larger: its pulses in parts, and
             // what does not qualify in bands of tile rows
             const Band w = window(r, std::min(length, r + sr));
-            if (part < 64 || sp.group_strips < whole.strips_x) {
+            if (part < bp::kStripMinPulses) {
+                // the budget holds no window that a strip qualifies with
                 sp.lines = false;
                 break;
             }
@@ -1865,13 +1867,16 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
                 bp::LineArgs la = sp.la;
                 la.batch = batch_b;
                 la.rc = rc_base;
-                la.s_begin = 0;
-                la.s_end = band_strips[b];
                 la.q_begin = bd.k0 / 64 * 64;
                 la.q_end = bd.k1;
                 la.q_first = bd.first;
-                la.carry = static_cast<double2*>(hp.carry.ptr);
-                BP_HIP_CHECK(bp::launch_strips(la, sp.width, bd.last, s));
+                for (int64_t s0 = 0; s0 < band_strips[b]; s0 += sp.group_strips) {
+                    la.s_begin = s0;
+                    la.s_end = std::min(band_strips[b], s0 + sp.group_strips);
+                    la.carry = reinterpret_cast<double2*>(static_cast<unsigned char*>(hp.carry.ptr) +
+                                                          bp::line_carry_bytes() * s0);
+                    BP_HIP_CHECK(bp::launch_strips(la, sp.width, bd.last, s));
+                }
             } else if ((rc = enqueue_sum(sp, batch_b, rc_base, band_groups[b],
                                          bd.kind == Band::kTiles ? 0 : band_strips[b], s))) {
                 return rc;

@@ -188,6 +188,9 @@ constexpr int kEndDegree = 4;        // weights of the taps at a cell's end
 // Limits a strip has to keep, at the ends of its lines' common pulses:
 constexpr float kLineMaxShift = 0.33f;   // bins between a line and the reference line
 constexpr double kLineMaxSlope = 1.0;    // cycles per pulse
+// Pulses of each of its pixels, at least: with fewer the pixel-by-pixel sum is
+// short anyway, and host pulses in parts of whole chunks need as many.
+constexpr int kStripMinPulses = 64;
 // phase (rad) a line gathers over half a chunk against the reference line,
 // plus pi times its bins off: what the 6 or 8 nodes interpolate (the residue
 // is x^N / (N! 2^(N-1)) at most: 1.5e-4 for x = 2.4 and N = 8, 1.2e-4 for x =

@@ -48,7 +48,7 @@
 // derivatives at four of the nodes, in such strips only, bring that in to
 // first order (24 % more work in the nodes).
 //
-// A strip qualifies when every pixel integrates pulses, no tap leaves the
+// A strip qualifies when every pixel integrates 64 pulses, no tap leaves the
 // range line, lines differ by at most 0.33 bin and the phase bounds of
 // bp_internal.h, the nodes reproduce every line's phase slope, and the
 // columns' fractional bins agree (corrections would otherwise be needed at
@@ -290,7 +290,7 @@ void strip_fit_kernel(GeomArgs a, LineArgs l)
         const int i = wave * 8 + q;
         if (i >= st.h) break;
         const PixGeom& g = a.geom[st.rec + i * st.width + col];
-        ok &= g.status == kPixOk && g.kstop > g.kstart;
+        ok &= g.status == kPixOk && g.kstop - g.kstart >= kStripMinPulses;
         lo = min(lo, g.kstart);
         hi = max(hi, g.kstop);
         flo = max(flo, g.kstart);

@@ -152,3 +152,24 @@ def test_few_and_many_strips_agree(torch_gpu, width, tropo):
                     tropo, precision="split")
         outs.append(out)
     np.testing.assert_array_equal(outs[0][:64], outs[1])
+
+
+def test_budget_below_any_strip_window(torch_gpu):
+    """Windows of about 45 pulses under a budget of 63: no strip qualifies with
+    fewer than 64, so host pulses in bands of tile rows still give the resident
+    call's result to the bit."""
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import LUT2d
+    from isce3_amd.focus import backproject
+    orb, in_geom, dem, raw, kernel = _scene(8)
+    og = RadarGeometry(sim._grid(-0.5 * 130 / sim.PRF, sim.PRF, sim.R0 + 40 * sim.DR, sim.DR, 130, 70),
+                       orb, LUT2d())
+    outs = []
+    for pulses in (NA, 63):
+        out = np.empty((130, 70), np.complex64)
+        backproject(out, og, raw, in_geom, dem, sim.FC, 500.0, kernel, "nodelay",
+                    precision="split", max_window_bytes=pulses * NR * 8)
+        outs.append(out)
+    np.testing.assert_array_equal(outs[1], outs[0])
+    assert np.isfinite(outs[0]).all()
