@@ -1984,8 +1984,7 @@ struct bp_scene {
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     std::vector<int> block_of_grid;
     LinePlan lines{};          // line-interpolated sum (lane_rows 2)
-    int64_t line_strips = 0;   // strips the scene holds records for, ...
-    int64_t line_group = 0;    // ... and workspace for at a time
+    int64_t line_group = 0;    // strips the scene holds workspace for at a time
     int64_t part_records = 0;  // plain: pixels whose segment sums the scene holds
     // A kernel node whose grid follows the batch, with its captured launch
     // parameters: the geometry pass (geometry groups), fit and plain sum (tile
@@ -2002,6 +2001,7 @@ struct bp_scene {
     struct Graph {
         int chunk, blocks_per_cu, lane_rows;
         bool staged;
+        int64_t groups;   // of line_group strips, 0 without the line-interpolated sum
         hipGraph_t graph;
         hipGraphExec_t exec;
         std::vector<GridNode> nodes;
@@ -2020,17 +2020,6 @@ void destroy_graphs(bp_scene* sc)
     sc->graphs.clear();
 }
 
-// Room for n strips (the graphs hold the buffers' addresses: a scene that
-// grows captures them anew).
-void scene_lines(bp_scene* sc, int64_t n)
-{
-    if (!sc->lines.on || n <= sc->line_strips) return;
-    destroy_graphs(sc);
-    sc->line_strips = n;
-    sc->line_group = alloc_lines(sc->lines, n, sc->sc);
-    if (sc->line_group == 0) sc->lines.on = false;
-}
-
 void destroy_scene(bp_scene* sc)
 {
     destroy_graphs(sc);
@@ -2044,15 +2033,31 @@ void destroy_scene(bp_scene* sc)
     delete sc;
 }
 
-// Capture the step of one launch configuration.
-int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
+// Strips of max_pixels pixels in max_blocks blocks at most: a block of l x w
+// pixels has ceil(l / rows) ceil(w / 64) <= l w / rows + 1, rows <= 64.
+int64_t most_strips(int64_t max_pixels, int max_blocks, int rows)
+{
+    return max_pixels / rows + std::min<int64_t>(max_blocks, max_pixels);
+}
+
+// ... and those that a scene has workspace for at a time: more than blocks of
+// some hundred pixels a side need; narrower ones run in groups.
+int64_t scene_strips(int64_t max_pixels, int max_blocks, int rows)
+{
+    return std::min(most_strips(max_pixels, max_blocks, rows),
+                    max_pixels / (rows * 64) * 5 / 4 + 2 * std::min(max_blocks, 64) + 8);
+}
+
+// Capture the step of one launch configuration, for up to `groups` groups of
+// strips.
+int capture_graph(bp_scene* sc, const Opts& o, int64_t groups, bp_scene::Graph* out)
 {
     bp_context* c = sc->ctx;
     Step sp;
     build_step(sp, sc->st, sc->sc, sc->args, sc->width, o, c->n_cu);
-    if (sc->lines.on && o.lane_rows == 2 && !o.staged) {
-        set_lines(sp, sc->lines, sc->sc, sc->args, sc->line_strips, sc->line_group);
-        if (sp.la.few == 0) sp.la.few = 2;   // replayed with any count up to line_strips
+    if (groups > 0) {
+        set_lines(sp, sc->lines, sc->sc, sc->args, groups * sc->line_group, sc->line_group);
+        if (sp.la.few == 0) sp.la.few = 2;   // replayed with any count up to the groups'
     }
     if (sc->part_records > 0) {
         sp.sa.parts = static_cast<double2*>(sc->sc.parts.ptr);
@@ -2129,10 +2134,8 @@ int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
             }
         }
     }
-    const size_t groups =
-        sp.lines ? (size_t)((sp.n_strips + sp.group_strips - 1) / sp.group_strips) : 0;
     const size_t per_group = sp.lines && sp.la.few == 2 ? 5 : 4;
-    const size_t want = 2 + (total_fn ? 1 : 0) + (sp.lines ? 1 + per_group * groups : 0);
+    const size_t want = 2 + (total_fn ? 1 : 0) + (sp.lines ? 1 + per_group * (size_t)groups : 0);
     if (out->nodes.size() != want) {
         (void)hipGraphDestroy(g);
         return fail(BP_ERR_HIP, "captured step is missing its kernel nodes");
@@ -2147,6 +2150,7 @@ int capture_graph(bp_scene* sc, const Opts& o, bp_scene::Graph* out)
     out->blocks_per_cu = o.blocks_per_cu;
     out->lane_rows = o.lane_rows;
     out->staged = o.staged;
+    out->groups = groups;
     out->graph = g;
     out->exec = x;
     return BP_SUCCESS;
@@ -2225,9 +2229,14 @@ try {
         Opts two{};
         two.lane_rows = 2;
         sc->lines = plan_lines(sc->args, width, two);
-        // strips of square blocks; a call of narrower ones grows the scene
-        scene_lines(sc, max_pixels / (bp::kStripLines * 64) * 5 / 4 +
-                            2 * std::min(max_blocks, 64) + 8);
+        if (sc->lines.on) {
+            const int64_t n = scene_strips(max_pixels, max_blocks, sc->lines.rows);
+            if (ensure(sc->sc.strips, sizeof(bp::StripInfo) *
+                                          most_strips(max_pixels, max_blocks, sc->lines.rows)) ==
+                BP_SUCCESS)
+                sc->line_group = alloc_lines(sc->lines, n, sc->sc);
+            sc->lines.on = sc->line_group > 0;
+        }
     }
     int32_t oor = 0;
     if (hipMemcpyAsync(&oor, static_cast<int32_t*>(sc->sc.flags.ptr) + 1, sizeof(oor),
@@ -2280,8 +2289,9 @@ try {
     if (npix == 0) return BP_SUCCESS;
     BP_HIP_CHECK(hipSetDevice(sc->ctx->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool lines = sc->lines.on && o.lane_rows == 2 && !o.staged;
-    if (lines) {
+    // strips in groups of the scene's workspace; graphs for powers of two of them
+    int64_t groups = 0;
+    if (sc->lines.on && o.lane_rows == 2 && !o.staged) {
         o.strip_rows = sc->lines.rows;
         int64_t n_strips = 0;
         for (int b = 0; b < n_blocks; ++b) {
@@ -2290,17 +2300,17 @@ try {
             d.map.width = blocks[b].grid.width;
             if (d.map.length * d.map.width > 0) n_strips += map_strips(d, o.strip_rows);
         }
-        scene_lines(sc, n_strips);
+        for (groups = 1; groups * sc->line_group < n_strips;) groups *= 2;
     }
 
     bp_scene::Graph* g = nullptr;
     for (auto& x : sc->graphs)
         if (x.chunk == o.chunk && x.blocks_per_cu == o.blocks_per_cu && x.staged == o.staged &&
-            x.lane_rows == o.lane_rows)
+            x.lane_rows == o.lane_rows && x.groups == groups)
             g = &x;
     if (g == nullptr) {
         bp_scene::Graph ng{};
-        if ((rc = capture_graph(sc, o, &ng)) != BP_SUCCESS) return rc;
+        if ((rc = capture_graph(sc, o, groups, &ng)) != BP_SUCCESS) return rc;
         sc->graphs.push_back(ng);
         g = &sc->graphs.back();
     }

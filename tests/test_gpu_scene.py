@@ -106,3 +106,39 @@ def test_scene_limits(torch_gpu):
         with pytest.raises(errors.InvalidArgument):
             scene.focus([o1, o2], [small, small])  # two blocks, one reserved
         assert scene.focus([o1], [small]) == [False]
+
+
+def test_strip_counts_without_allocation(torch_gpu):
+    """Replays of 40 strips, of one, of 640 narrow ones (more than the scene has
+    workspace for at a time: several groups in the graph) and of 40 again: the
+    eager results, and no device memory beyond a graph's own."""
+    from isce3_amd import sim
+    from isce3_amd.focus import Scene
+    torch = torch_gpu
+    sc = sim.make_scene("tiny")
+    na, nr = 1600, 2700
+    sc.in_grid = sim._grid(-0.5 * na / sim.PRF, sim.PRF, sim.R0, sim.DR, na, nr)
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(4)
+    raw_dev = torch.randn((na, nr), dtype=torch.complex64, device="cuda:0", generator=gen)
+
+    def block(rows, cols, c0):
+        return sim._grid(-0.5 * rows / sim.PRF, sim.PRF, sim.R0 + c0 * sim.DR, sim.DR, rows, cols)
+
+    batches = [[block(64, 40 * 64, 40)], [block(20, 33, 40)],
+               [block(1024, 1, 40 + 9 * i) for i in range(40)], [block(64, 40 * 64, 40)]]
+    with Scene(raw_dev, sc.in_geometry(), sc.orbit, sc.doppler, sc.dem, sc.fc, sc.ds, sc.kernel,
+               sc.dry_tropo_model, precision="split", max_pixels=40 * 4096, max_blocks=64) as scene:
+        refs = [eager(sc, raw_dev, b, "split", {}) for b in batches]
+        replay(scene, batches[1], {})
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info(0)[0]
+        for b, ref in zip(batches, refs):
+            print(f"[scene] {len(b)} blocks of {b[0].length} x {b[0].width}", flush=True)
+            outs, _, _, st = replay(scene, b, {}, heights=False)
+            for z, z0 in zip(outs, ref[0]):
+                np.testing.assert_array_equal(z, z0)
+            assert st["updates"] == ref[3]["updates"]
+        taken = free - torch.cuda.mem_get_info(0)[0]
+        print(f"[scene] {taken / 2 ** 20:.1f} MiB taken", flush=True)
+        assert taken <= 16 << 20
