@@ -190,9 +190,26 @@ const char* bp_last_error_message(void);
 
 /* Device scratch bytes per output pixel that a context holds for a call of
  * the given precision (per-pixel geometry records, plus the split-precision
- * records); a context grows its scratch to pixels x this value and keeps it.
+ * records); a context grows its scratch to pixels x this value and keeps it,
+ * beside the workspace below.
  * No reference counterpart: used by callers that budget device memory. */
 int64_t bp_scratch_bytes_per_pixel(int precision);
+
+/* Device workspace of the sums, at most, that a scene (scene nonzero) or a
+ * context (zero) holds beside that for up to max_pixels output pixels in up to
+ * max_blocks blocks: strips of the line-interpolated split sum (1.5 GiB and 32
+ * bytes per strip at most) or segment sums of the plain sum (256 MiB at most),
+ * with `limit` as in bp_context_limit_workspace.  Needs no device.  Negative:
+ * an error code. */
+int64_t bp_workspace_bytes(const bp_radar_geometry* in_geometry, double fc, double ds,
+                           const bp_kernel* kernel, int dry_tropo_model, int precision,
+                           int64_t max_pixels, int max_blocks, int scene, int64_t limit);
+
+/* Limit that workspace, for the calls made and scenes created on `ctx` from
+ * here on, to `bytes` (but no less than one strip takes), or lift the limit (a
+ * negative number, the default).  Results do not depend on it: strips run in
+ * smaller groups, segments in one wavefront. */
+int bp_context_limit_workspace(bp_context* ctx, int64_t bytes);
 
 /*
  * Focus in azimuth by time-domain backprojection.

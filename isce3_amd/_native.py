@@ -116,6 +116,9 @@ _SIGNATURES = {
     "bp_context_destroy": (C.c_int, [C.c_void_p]),
     "bp_last_error_message": (C.c_char_p, []),
     "bp_scratch_bytes_per_pixel": (C.c_int64, [C.c_int]),
+    "bp_workspace_bytes": (C.c_int64, [_P(RadarGeometry_t), C.c_double, C.c_double, _P(Kernel_t),
+                                       C.c_int, C.c_int, C.c_int64, C.c_int, C.c_int, C.c_int64]),
+    "bp_context_limit_workspace": (C.c_int, [C.c_void_p, C.c_int64]),
     "bp_backproject": (C.c_int, [C.c_void_p, _P(RadarGeometry_t), _P(RadarGeometry_t), _P(Dem_t),
                                  C.c_double, C.c_double, _P(Kernel_t), C.c_int,
                                  _P(Rdr2GeoParams_t), _P(Geo2RdrParams_t), C.c_void_p,

@@ -139,6 +139,7 @@ struct HostPath {
 struct bp_context {
     int device = 0;
     int n_cu = 0;
+    int64_t workspace_limit = -1;      // bp_context_limit_workspace
     unsigned char* scratch = nullptr;  // device address of this device's no-alloc scratch
     std::string scratch_err;           // why it is null
     StaticData st;
@@ -708,6 +709,13 @@ void free_host_path(HostPath& h)
 
 }  // namespace
 
+extern "C" int bp_context_limit_workspace(bp_context* c, int64_t bytes)
+{
+    if (c == nullptr) return fail(BP_ERR_INVALID_ARGUMENT, "null argument");
+    c->workspace_limit = bytes < 0 ? -1 : bytes;
+    return BP_SUCCESS;
+}
+
 extern "C" int bp_context_destroy(bp_context* c)
 try {
     if (c == nullptr) return BP_SUCCESS;
@@ -1072,28 +1080,64 @@ LinePlan plan_lines(const CallArgs& a, int width, const Opts& o)
 constexpr int64_t kPlainWaves = 16384;
 constexpr size_t kPartBytes = size_t(256) << 20;
 
-int plain_segments(const CallArgs& a, int64_t n_seq, int64_t n_rec)
+// The lesser of a workspace bound and the context's own limit (none below 0).
+size_t limited(size_t bytes, int64_t limit)
+{
+    return limit < 0 ? bytes : std::min(bytes, (size_t)limit);
+}
+
+int plain_segments(const CallArgs& a, int64_t n_seq, int64_t n_rec, int64_t limit)
 {
     if (a.precision != BP_PRECISION_PLAIN || n_seq >= kPlainWaves) return 0;
     const int64_t segs = (a.in_geometry->grid.length + bp::kPlainSeg - 1) / bp::kPlainSeg;
-    if (segs < 2 || segs > 65535 || (double)segs * n_rec * sizeof(double2) > (double)kPartBytes)
+    if (segs < 2 || segs > 65535 ||
+        (double)segs * n_rec * sizeof(double2) > (double)limited(kPartBytes, limit))
         return 0;
     return (int)segs;
 }
 
-// Strips whose workspace a call with n of them takes at once.
-int64_t line_group(const LinePlan& p, int64_t n)
+// Pixels whose segment sums a scene holds (0: no segments of their own).
+int64_t scene_part_records(const CallArgs& a, int64_t max_pixels, int64_t limit)
 {
-    return std::min<int64_t>(n, (int64_t)(kLineBytes / p.strip_bytes));
+    const int64_t length = a.in_geometry->grid.length;
+    if (a.precision != BP_PRECISION_PLAIN || length <= bp::kPlainSeg) return 0;
+    const int64_t segs = (length + bp::kPlainSeg - 1) / bp::kPlainSeg;
+    return std::min({max_pixels, kPlainWaves * 64,
+                     (int64_t)(limited(kPartBytes, limit) / (segs * sizeof(double2)))});
 }
 
-// Workspace for n strips, as many at once as the device has room for: their
-// number.  Results do not depend on it, but for a device without room for a
-// single strip (0.3 to 0.5 MB), where the call sums pixel by pixel (0).
-int64_t alloc_lines(const LinePlan& p, int64_t n, Scratch& sc)
+// Strips of max_pixels pixels in max_blocks blocks at most: a block of l x w
+// pixels has ceil(l / rows) ceil(w / 64) <= l w / rows + 1, rows <= 64.
+int64_t most_strips(int64_t max_pixels, int max_blocks, int rows)
 {
-    if (ensure(sc.strips, sizeof(bp::StripInfo) * n) != BP_SUCCESS) return 0;
-    for (int64_t group = line_group(p, n); group > 0; group /= 2)
+    return max_pixels / rows + std::min<int64_t>(max_blocks, max_pixels);
+}
+
+// ... and those that a scene has workspace for at a time: more than blocks of
+// some hundred pixels a side need; narrower ones run in groups.
+int64_t scene_strips(int64_t max_pixels, int max_blocks, int rows)
+{
+    return std::min(most_strips(max_pixels, max_blocks, rows),
+                    max_pixels / (rows * 64) * 5 / 4 + 2 * std::min(max_blocks, 64) + 8);
+}
+
+// Strips whose workspace is taken at once for n of them, beside the StripInfo
+// of `records` strips.
+int64_t line_group(const LinePlan& p, int64_t n, int64_t records, int64_t limit)
+{
+    const int64_t left = (int64_t)limited(kLineBytes, limit) -
+                         (limit < 0 ? 0 : (int64_t)sizeof(bp::StripInfo) * records);
+    return std::min<int64_t>(n, std::max<int64_t>(left / (int64_t)p.strip_bytes, 1));
+}
+
+// StripInfo for `records` strips and workspace for n, or as many of them at once
+// as limit and device have room for: their number.  Results do not depend on
+// it, but for a device without room for a single strip (0.3 to 0.5 MB), where the
+// call sums pixel by pixel (0).
+int64_t alloc_lines(const LinePlan& p, int64_t n, int64_t records, int64_t limit, Scratch& sc)
+{
+    if (ensure(sc.strips, sizeof(bp::StripInfo) * records) != BP_SUCCESS) return 0;
+    for (int64_t group = line_group(p, n, records, limit); group > 0; group /= 2)
         if (ensure(sc.lines, p.strip_bytes * group) == BP_SUCCESS) return group;
     return 0;
 }
@@ -1355,7 +1399,7 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
         return rc;
     const int64_t n_rec = npix;
 
-    int segs = plain_segments(a, hdr.n_seq, n_rec);
+    int segs = plain_segments(a, hdr.n_seq, n_rec, c->workspace_limit);
     if (segs > 0) {
         const size_t bytes = sizeof(double2) * (size_t)segs * n_rec;
         if (carve ? carve_parts(*carve, bytes, sc) : ensure(sc.parts, bytes)) segs = 0;
@@ -1372,7 +1416,7 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
         if (carve) {
             group = carve_lines(*carve, lp, hdr.n_strips, sc);
         } else {
-            group = alloc_lines(lp, hdr.n_strips, sc);
+            group = alloc_lines(lp, hdr.n_strips, hdr.n_strips, c->workspace_limit, sc);
         }
     }
     BP_HIP_CHECK(bp::launch_clear(static_cast<int32_t*>(sc.flags.ptr), n_flag, s));
@@ -1632,7 +1676,8 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
     if ((rc = ensure(c->sc.geom, sizeof(bp::PixGeom) * npix))) return rc;
     if (a.precision == BP_PRECISION_SPLIT && (rc = ensure(c->sc.split, sizeof(bp::PixSplit) * npix)))
         return rc;
-    const int64_t group = lp.on ? alloc_lines(lp, hdr.n_strips, c->sc) : 0;
+    const int64_t group =
+        lp.on ? alloc_lines(lp, hdr.n_strips, hdr.n_strips, c->workspace_limit, c->sc) : 0;
     BP_HIP_CHECK(bp::launch_clear(static_cast<int32_t*>(c->sc.flags.ptr), n_flag, s));
     if ((rc = pulse_states(c->st, a, static_cast<int32_t*>(c->sc.flags.ptr), s))) return rc;
 
@@ -1952,6 +1997,33 @@ try {
     return bp_host_exception();
 }
 
+extern "C" int64_t bp_workspace_bytes(const bp_radar_geometry* ig, double fc, double ds,
+                                      const bp_kernel* kernel, int dry_tropo_model, int precision,
+                                      int64_t max_pixels, int max_blocks, int scene, int64_t limit)
+try {
+    // the rules of check_call that the plans below rely on
+    if (ig == nullptr || kernel == nullptr || !(ig->grid.prf > 0) || !(fc > 0) || !(ds > 0) ||
+        kernel->n < 2 || kernel->table == nullptr || !(kernel->halfwidth > 0) || ig->orbit.n < 2 ||
+        ig->orbit.pos == nullptr || ig->orbit.vel == nullptr || max_pixels < 1 || max_blocks < 1)
+        return fail(BP_ERR_INVALID_ARGUMENT, "invalid argument");
+    CallArgs a{nullptr, nullptr, ig, nullptr, fc, ds, kernel, dry_tropo_model, nullptr, nullptr,
+               nullptr, precision};
+    if (precision == BP_PRECISION_PLAIN) {
+        const int64_t segs = (ig->grid.length + bp::kPlainSeg - 1) / bp::kPlainSeg;
+        return scene_part_records(a, max_pixels, limit) * segs * (int64_t)sizeof(double2);
+    }
+    Opts two{};
+    two.lane_rows = 2;
+    const LinePlan p = plan_lines(a, (int)std::ceil(2.0 * kernel->halfwidth), two);
+    if (!p.on) return 0;
+    const int64_t most = most_strips(max_pixels, max_blocks, p.rows);
+    const int64_t n = scene ? scene_strips(max_pixels, max_blocks, p.rows) : most;
+    return (int64_t)sizeof(bp::StripInfo) * most +
+           (int64_t)p.strip_bytes * line_group(p, n, most, limit);
+} catch (...) {
+    return bp_host_exception();
+}
+
 // ------------------------------------------------------------------ scenes
 
 // One raw set kept resident with everything its tile requests share, scratch
@@ -2031,21 +2103,6 @@ void destroy_scene(bp_scene* sc)
         if (ev) (void)hipEventDestroy(ev);
     if (sc->cap) (void)hipStreamDestroy(sc->cap);
     delete sc;
-}
-
-// Strips of max_pixels pixels in max_blocks blocks at most: a block of l x w
-// pixels has ceil(l / rows) ceil(w / 64) <= l w / rows + 1, rows <= 64.
-int64_t most_strips(int64_t max_pixels, int max_blocks, int rows)
-{
-    return max_pixels / rows + std::min<int64_t>(max_blocks, max_pixels);
-}
-
-// ... and those that a scene has workspace for at a time: more than blocks of
-// some hundred pixels a side need; narrower ones run in groups.
-int64_t scene_strips(int64_t max_pixels, int max_blocks, int rows)
-{
-    return std::min(most_strips(max_pixels, max_blocks, rows),
-                    max_pixels / (rows * 64) * 5 / 4 + 2 * std::min(max_blocks, 64) + 8);
 }
 
 // Capture the step of one launch configuration, for up to `groups` groups of
@@ -2218,25 +2275,19 @@ try {
     if (hipMemsetAsync(sc->sc.flags.ptr, 0, flag_bytes, s) != hipSuccess)
         return bail(fail(BP_ERR_HIP, "hipMemsetAsync failed"));
     if ((rc = pulse_states(sc->st, sc->args, static_cast<int32_t*>(sc->sc.flags.ptr), s))) return bail(rc);
-    if (precision == BP_PRECISION_PLAIN && in_geometry->grid.length > bp::kPlainSeg) {
+    if (const int64_t n = scene_part_records(sc->args, max_pixels, c->workspace_limit)) {
         const int64_t segs = (in_geometry->grid.length + bp::kPlainSeg - 1) / bp::kPlainSeg;
-        const int64_t most = (int64_t)(kPartBytes / (segs * sizeof(double2)));
-        const int64_t n = std::min(max_pixels, std::min(most, kPlainWaves * 64));
-        if (n > 0 && ensure(sc->sc.parts, sizeof(double2) * segs * n) == BP_SUCCESS)
-            sc->part_records = n;
+        if (ensure(sc->sc.parts, sizeof(double2) * segs * n) == BP_SUCCESS) sc->part_records = n;
     }
     {
         Opts two{};
         two.lane_rows = 2;
         sc->lines = plan_lines(sc->args, width, two);
-        if (sc->lines.on) {
-            const int64_t n = scene_strips(max_pixels, max_blocks, sc->lines.rows);
-            if (ensure(sc->sc.strips, sizeof(bp::StripInfo) *
-                                          most_strips(max_pixels, max_blocks, sc->lines.rows)) ==
-                BP_SUCCESS)
-                sc->line_group = alloc_lines(sc->lines, n, sc->sc);
-            sc->lines.on = sc->line_group > 0;
-        }
+        if (sc->lines.on)
+            sc->line_group = alloc_lines(sc->lines, scene_strips(max_pixels, max_blocks, sc->lines.rows),
+                                         most_strips(max_pixels, max_blocks, sc->lines.rows),
+                                         c->workspace_limit, sc->sc);
+        sc->lines.on = sc->line_group > 0;
     }
     int32_t oor = 0;
     if (hipMemcpyAsync(&oor, static_cast<int32_t*>(sc->sc.flags.ptr) + 1, sizeof(oor),
@@ -2321,7 +2372,7 @@ try {
                          sc->h_desc, sc->max_blocks, &hdr, sc->block_of_grid)) != BP_SUCCESS)
         return rc;
     if (sc->part_records > 0 && npix <= sc->part_records) {
-        hdr.plain_segs = plain_segments(sc->args, hdr.n_seq, npix);
+        hdr.plain_segs = plain_segments(sc->args, hdr.n_seq, npix, -1);
         std::memcpy(sc->h_desc, &hdr, sizeof(hdr));
     }
     for (const bp_scene::GridNode& gn : g->nodes) {

@@ -478,7 +478,7 @@ class Scene:
                  dem: DEMInterpolator, fc: float, ds: float, kernel: KernelF32,
                  dry_tropo_model: str = "tsx", rdr2geo_params: Optional[dict] = None,
                  geo2rdr_params: Optional[dict] = None, *, precision: str = "split",
-                 max_pixels: int = 1 << 22, max_blocks: int = 64):
+                 max_pixels: int = 1 << 22, max_blocks: int = 64, _context=None):
         self._h = None
         if precision not in _PRECISION:
             raise errors.InvalidArgument(f"precision must be 'plain' or 'split', got {precision!r}")
@@ -509,7 +509,7 @@ class Scene:
         g2r = parse_geo2rdr_params(geo2rdr_params or {})
         h = C.c_void_p()
         with torch.cuda.device(self.device):
-            ctx = _contexts.get(self.device)
+            ctx = _contexts.get(self.device) if _context is None else _context
             _keep = (in_geometry, out_orbit, out_doppler, dem, kernel)
             rc = _native.lib().bp_scene_create(
                 ctx, C.byref(oorb), C.byref(odop), C.byref(ig), C.byref(dm), float(fc),

@@ -20,9 +20,11 @@ while other batches run join the next batch, and batches of different
 workers overlap on the device.  The ``fcfs`` policy (one worker, one request
 per batch) is the first-come-first-served baseline.
 
-Memory accounting: the resident raw sets and each worker's per-pixel scratch
+Memory accounting: the resident raw sets, each worker's per-pixel scratch
 (sized for ``max_batch_pixels``, one copy per raw set when the executor keeps
-a resident scene per set) are charged once at construction; every admitted
+a resident scene per set) and its workspace of the sums are charged once at
+construction; where the budget is short, the workspace is limited to what it
+leaves beside one full batch's outputs.  Every admitted
 request is charged its output bytes until it is released (at once when
 ``keep_outputs`` is false, else by ``Request.release``).
 """
@@ -130,14 +132,33 @@ class GpuExecutor:
         self._workers = {}
         self._scenes = {}
         self._limits = (1 << 24, 256)
+        self._workspace = -1
 
     def scratch_copies(self, n_sets: int) -> int:
         """Per-pixel scratch buffers each worker holds (one per raw set when
         every set has its own scene)."""
         return n_sets if self.graphs else 1
 
-    def configure(self, max_batch_pixels: int, max_batch_requests: int):
+    def workspace_bytes(self, sets, precision: str, max_batch_pixels: int,
+                        max_batch_requests: int, limit: int = -1) -> int:
+        """Workspace of the sums each worker holds (bp_workspace_bytes): of all
+        its scenes, or of its context, which grows to the largest set's."""
+        from .focus import _PRECISION, geometry_struct, parse_dry_tropo_model
+        sizes = []
+        for raw in sets:
+            ig, kr = geometry_struct(raw.in_geometry), raw.kernel._struct()
+            n = _native.lib().bp_workspace_bytes(
+                C.byref(ig), float(raw.fc), float(raw.ds), C.byref(kr),
+                parse_dry_tropo_model(raw.dry_tropo_model), _PRECISION[precision],
+                int(max_batch_pixels), int(max_batch_requests), int(self.graphs), int(limit))
+            _native.check(min(n, 0))
+            sizes.append(n)
+        return sum(sizes) if self.graphs else max(sizes, default=0)
+
+    def configure(self, max_batch_pixels: int, max_batch_requests: int, workspace: int = -1):
+        """Limits of a batch, and of each scene's or context's workspace (-1: none)."""
         self._limits = (int(max_batch_pixels), int(max_batch_requests))
+        self._workspace = int(workspace)
 
     def start_worker(self, index: int):
         torch = self.torch
@@ -145,6 +166,7 @@ class GpuExecutor:
             stream = torch.cuda.Stream(device=self.device)  # default priority
         h = C.c_void_p()
         _native.check(_native.lib().bp_context_create(self.device, C.byref(h)))
+        _native.check(_native.lib().bp_context_limit_workspace(h, self._workspace))
         self._workers[index] = (stream, h)
 
     def stop_worker(self, index: int):
@@ -161,7 +183,7 @@ class GpuExecutor:
             sc = Scene(raw.signal, raw.in_geometry, raw.out_orbit, raw.out_doppler, raw.dem,
                        raw.fc, raw.ds, raw.kernel, raw.dry_tropo_model, raw.rdr2geo_params,
                        raw.geo2rdr_params, precision=precision, max_pixels=self._limits[0],
-                       max_blocks=self._limits[1])
+                       max_blocks=self._limits[1], _context=self._workers[index][1])
             self._scenes[key] = sc
         return sc
 
@@ -245,6 +267,17 @@ class Server:
             raise errors.InvalidArgument(
                 f"resident sets and worker scratch ({self.base_bytes} B) exceed the budget "
                 f"({self.budget_bytes} B)")
+        workspace = -1
+        if hasattr(self.executor, "workspace_bytes"):
+            spare = max(0, self.budget_bytes - self.base_bytes -
+                        self.max_batch_pixels * OUT_BYTES_PER_PIXEL)
+            args = (self.sets, precision, self.max_batch_pixels, self.max_batch_requests)
+            held = self.workers * self.executor.workspace_bytes(*args)
+            if held > spare:
+                # every request that fits the budget without it still does
+                workspace = spare // (self.workers * max(copies, 1))
+                held = min(self.workers * self.executor.workspace_bytes(*args, workspace), spare)
+            self.base_bytes += held
         self.in_use = self.base_bytes
         self.peak_in_use = self.base_bytes
         self._cv = threading.Condition()
@@ -255,7 +288,8 @@ class Server:
         self._batch_seq = 0
         self.batches: List[dict] = []
         if hasattr(self.executor, "configure"):
-            self.executor.configure(self.max_batch_pixels, self.max_batch_requests)
+            limits = (self.max_batch_pixels, self.max_batch_requests)
+            self.executor.configure(*limits, *([workspace] if workspace >= 0 else []))
         self._threads = []
         for i in range(self.workers):
             self.executor.start_worker(i)

@@ -142,3 +142,41 @@ def test_strip_counts_without_allocation(torch_gpu):
         taken = free - torch.cuda.mem_get_info(0)[0]
         print(f"[scene] {taken / 2 ** 20:.1f} MiB taken", flush=True)
         assert taken <= 16 << 20
+
+
+@pytest.mark.parametrize("precision,limit", [("split", -1), ("split", 20 << 20), ("plain", -1)])
+def test_memory_held_as_stated(torch_gpu, precision, limit):
+    """A scene takes at most its per-pixel scratch and bp_workspace_bytes (and
+    some MiB of tables and allocation granules), and a limit does not change
+    results."""
+    import ctypes as C
+    from isce3_amd import _native
+    from isce3_amd.focus import _PRECISION, Scene, geometry_struct
+    torch = torch_gpu
+    sc, raw = scene_and_raw("small")
+    raw_dev = torch.from_numpy(raw.copy()).cuda()
+    grids = uneven_blocks(sc)
+    ref = eager(sc, raw_dev, grids, precision, {})
+    ctx = C.c_void_p()
+    lib = _native.lib()
+    _native.check(lib.bp_context_create(0, C.byref(ctx)))
+    _native.check(lib.bp_context_limit_workspace(ctx, limit))
+    max_pixels = 1 << 20
+    geometry = sc.in_geometry()
+    ig, kr = geometry_struct(geometry), sc.kernel._struct()
+    said = max_pixels * lib.bp_scratch_bytes_per_pixel(_PRECISION[precision]) + \
+        lib.bp_workspace_bytes(C.byref(ig), sc.fc, sc.ds, C.byref(kr), 1, _PRECISION[precision],
+                               max_pixels, 16, 1, limit)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info(0)[0]
+    with Scene(raw_dev, sc.in_geometry(), sc.orbit, sc.doppler, sc.dem, sc.fc, sc.ds, sc.kernel,
+               sc.dry_tropo_model, precision=precision, max_pixels=max_pixels, max_blocks=16,
+               _context=ctx) as scene:
+        taken = free - torch.cuda.mem_get_info(0)[0]
+        print(f"[scene] {precision} limit {limit}: {taken / 2 ** 20:.1f} MiB, stated "
+              f"{said / 2 ** 20:.1f}", flush=True)
+        assert taken <= said + (24 << 20)
+        outs = replay(scene, grids, {}, heights=False)[0]
+        for z, z0 in zip(outs, ref[0]):
+            np.testing.assert_array_equal(z, z0)
+    lib.bp_context_destroy(ctx)

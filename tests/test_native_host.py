@@ -213,6 +213,31 @@ def test_scratch_bytes_match_the_server_accounting():
         serve.RECORD_BYTES_PER_PIXEL["split"]
 
 
+@pytest.mark.parametrize("precision,width,max_pixels,least,most", [
+    ("split", 8, 1 << 24, 1 << 30, (3 << 29) + (1 << 24)), ("split", 9, 1 << 16, 1 << 20, 156 * 700000),
+    ("split", 6, 1 << 24, 0, 0), ("plain", 8, 1 << 24, 128 << 20, 256 << 20),
+    ("plain", 8, 4096, 1, 16 << 20)])
+def test_workspace_bytes(precision, width, max_pixels, least, most):
+    """What a scene's sums hold beside its records, without and with a limit
+    (2^16 pixels in 64 blocks: workspace for 156 strips)."""
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.focus import _PRECISION, geometry_struct
+    grid = sim._grid(-2.5, sim.PRF, sim.R0, sim.DR, 8192, 16384)
+    geometry = RadarGeometry(grid, sim.straight_orbit(), core.LUT2d())
+    kernel = core.TabulatedKernelF32(core.KnabKernel(float(width), 0.8), 2048)
+    ig, kr = geometry_struct(geometry), kernel._struct()
+
+    def held(limit, scene=1):
+        return _native.lib().bp_workspace_bytes(C.byref(ig), sim.FC, 6.0, C.byref(kr), 1,
+                                                _PRECISION[precision], max_pixels, 64, scene, limit)
+
+    assert least <= held(-1) <= most
+    assert held(-1) <= held(-1, 0) <= (3 << 29) + (9 << 20)   # a context's calls of any shape
+    assert held(10 << 20) <= max(10 << 20, (9 << 20) + (1 << 20))
+    assert held(0) <= (9 << 20) + (1 << 20)     # 32 bytes a strip, and one strip
+
+
 def test_sincos_turns_against_long_double():
     """The plain sum's FP64 phase rotation: sin/cos of 2 pi t for t in turns
     agree with an extended-precision evaluation to a few ulp, over the

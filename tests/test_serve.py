@@ -242,3 +242,36 @@ def test_submit_many_lands_in_one_batch():
         r.wait(5)
     srv.close()
     assert [c["tags"] for c in ex.calls] == [list(range(6))]
+
+
+class WorkspaceExecutor(FakeExecutor):
+    """Holds `need` bytes of workspace per worker and raw set, or its limit."""
+    need = 10 ** 6
+
+    def scratch_copies(self, n_sets):
+        return n_sets
+
+    def workspace_bytes(self, sets, precision, pixels, requests, limit=-1):
+        return len(sets) * (self.need if limit < 0 else min(self.need, limit))
+
+    def configure(self, pixels, requests, workspace=-1):
+        self.workspace = workspace
+
+
+@pytest.mark.parametrize("spare,limit", [(10 ** 7, -1), (4 * 10 ** 6, -1), (3 * 10 ** 6, 750000),
+                                         (0, 0)])
+def test_workspace_charged_within_the_budget(spare, limit):
+    """Two workers' workspaces for two raw sets are charged; a budget that is
+    short of them limits them and still admits the largest request."""
+    base = 2 * 10 ** 6 + 2 * 2 * SCRATCH
+    largest = 4096 * serve.OUT_BYTES_PER_PIXEL
+    ref = [None]
+    ex = WorkspaceExecutor(ref)
+    srv = serve.Server([FakeSet(10 ** 6)] * 2, budget_bytes=base + largest + spare, workers=2,
+                       max_batch_pixels=4096, executor=ex)
+    ref[0] = srv
+    assert srv.base_bytes == base + min(4 * 10 ** 6, spare)
+    assert ex.workspace == limit
+    srv.submit(serve.Request(0, grid(64))).wait(5)
+    assert srv.peak_in_use <= srv.budget_bytes
+    srv.close()
