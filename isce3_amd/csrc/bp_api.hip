@@ -431,58 +431,84 @@ void build_pair_table(const bp_kernel& k, int W, std::vector<float>& out)
     }
 }
 
-// Least-squares polynomial of degree D (monomial coefficients) through
-// weighted samples of [-F, F], solved in the Chebyshev basis.
+// Least-squares polynomials of degree D over [-F, F] through samples at x with
+// weights w, solved in the Chebyshev basis: the matrix [D + 1][samples] that
+// takes the samples to the monomial coefficients.
 template<int D>
-void fit_polynomial(double F, const std::vector<double>& x, const std::vector<double>& y,
-                    const std::vector<double>& w, double* c)
+std::vector<double> polynomial_map(double F, const std::vector<double>& x,
+                                   const std::vector<double>& w)
 {
     constexpr int N = D + 1;
-    long double m[N][N + 1] = {};
-    for (size_t i = 0; i < x.size(); ++i) {
+    const int M = (int)x.size();
+    std::vector<long double> row[N];   // normal matrix, then a right side per sample
+    for (auto& r : row) r.assign(N + M, 0.L);
+    for (int i = 0; i < M; ++i) {
         long double t[N];
         t[0] = 1.;
         if (N > 1) t[1] = x[i] / F;
         for (int k = 2; k < N; ++k) t[k] = 2 * (x[i] / F) * t[k - 1] - t[k - 2];
         for (int r = 0; r < N; ++r) {
-            for (int q = 0; q < N; ++q) m[r][q] += w[i] * t[r] * t[q];
-            m[r][N] += w[i] * t[r] * y[i];
+            for (int q = 0; q < N; ++q) row[r][q] += w[i] * t[r] * t[q];
+            row[r][N + i] = w[i] * t[r];
         }
     }
     for (int k = 0; k < N; ++k) {
         int piv = k;
         for (int r = k + 1; r < N; ++r)
-            if (std::fabs(m[r][k]) > std::fabs(m[piv][k])) piv = r;
-        for (int q = 0; q <= N; ++q) std::swap(m[k][q], m[piv][q]);
+            if (std::fabs(row[r][k]) > std::fabs(row[piv][k])) piv = r;
+        std::swap(row[k], row[piv]);
         for (int r = 0; r < N; ++r) {
             if (r == k) continue;
-            const long double f = m[r][k] / m[k][k];
-            for (int q = k; q <= N; ++q) m[r][q] -= f * m[k][q];
+            const long double f = row[r][k] / row[k][k];
+            for (int q = k; q < N + M; ++q) row[r][q] -= f * row[k][q];
         }
     }
     // Chebyshev -> monomial
-    long double out[N] = {}, t0[N] = {}, t1[N] = {};
-    t0[0] = 1.;
-    if (N > 1) t1[1] = 1.;
-    for (int k = 0; k < N; ++k) {
-        const long double a = m[k][N] / m[k][k];
-        const long double* t = k == 0 ? t0 : t1;
-        for (int n = 0; n < N; ++n) out[n] += a * t[n];
-        if (k >= 1) {
-            long double t2[N] = {};
-            for (int n = 0; n < N; ++n) t2[n] = (n > 0 ? 2 * t1[n - 1] : 0.L) - t0[n];
-            for (int n = 0; n < N; ++n) {
-                t0[n] = t1[n];
-                t1[n] = t2[n];
-            }
-        }
-    }
+    long double basis[N][N] = {};
+    basis[0][0] = 1.;
+    if (N > 1) basis[1][1] = 1.;
+    for (int k = 2; k < N; ++k)
+        for (int n = 0; n < N; ++n)
+            basis[k][n] = (n > 0 ? 2 * basis[k - 1][n - 1] : 0.L) - basis[k - 2][n];
+    std::vector<double> out((size_t)N * M);
     long double f = 1.;
     for (int n = 0; n < N; ++n) {
-        c[n] = (double)(out[n] * f);
+        for (int i = 0; i < M; ++i) {
+            long double c = 0.;
+            for (int k = 0; k < N; ++k) c += basis[k][n] * (row[k][N + i] / row[k][k]);
+            out[(size_t)n * M + i] = (double)(c * f);
+        }
         f /= F;
     }
+    return out;
 }
+
+// What build_line_table needs of the fits of one kernel width, the same for every
+// kernel (made once per process, as every call builds its kernel's table).
+template<int W>
+struct LineFits {
+    static constexpr int kTaps = (W + 1) / 2, kSamples = 97, kEndSamples = 33;
+    static constexpr int D = bp::line_degree(W);
+    static constexpr double F = 0.5 + (double)bp::kLineMaxShift, E = 0.5 * (double)bp::kLineMaxShift;
+    std::vector<double> x, xe, cell[kTaps], end;
+    LineFits() : x(kSamples), xe(kEndSamples)
+    {
+        std::vector<double> w(kSamples);
+        for (int i = 0; i < kSamples; ++i) x[i] = F * std::cos(M_PI * (i + 0.5) / kSamples);
+        for (int t = 0; t < kTaps; ++t) {
+            for (int i = 0; i < kSamples; ++i)
+                w[i] = std::fabs(t - 0.5 * (W - 1) - x[i]) <= 0.5 * W ? 1. : 1e-8;
+            cell[t] = polynomial_map<D>(F, x, w);
+        }
+        for (int i = 0; i < kEndSamples; ++i) xe[i] = E * std::cos(M_PI * (i + 0.5) / kEndSamples);
+        end = polynomial_map<bp::kEndDegree>(E, xe, std::vector<double>(kEndSamples, 1.));
+    }
+    static const LineFits& get()
+    {
+        static const LineFits fits;
+        return fits;
+    }
+};
 
 // Tap weight polynomials of the line-interpolated sum: tap t's weight at
 // position f of its cell (0 at the centre, the cell |f| <= 1/2) continued
@@ -492,82 +518,81 @@ void fit_polynomial(double F, const std::vector<double>& x, const std::vector<do
 // The limit, 1e-4 of the kernel's peak at the worst position, keeps the sum's
 // error below that of the pixel-by-pixel sum's weight table (5.4e-5 relative at
 // width 8, 1.2e-4 with white noise).
-bool build_line_table(const bp_kernel& k, int W, bp::LineArgs* a)
+template<int W>
+bool fit_line_table(const bp_kernel& k, bp::LineArgs* a)
 {
-    if ((W != 8 && W != 9) || 2.0 * k.halfwidth != (double)W) return false;
-    const double hw = k.halfwidth, F = 0.5 + (double)bp::kLineMaxShift;
-    const double dx = hw / (k.n - 1.0);
+    using Fits = LineFits<W>;
+    const Fits& fits = Fits::get();
+    const double hw = k.halfwidth;
+    const double dx = hw / (k.n - 1.0), rdx = 1.0 / dx;
     auto weight = [&](double ax) {
-        const int i = std::min((int)std::floor(ax / dx), k.n - 2);
-        return (double)k.table[i] + (ax / dx - i) * (double)(k.table[i + 1] - k.table[i]);
+        const int i = std::min((int)(ax * rdx), k.n - 2);
+        return (double)k.table[i] + (ax * rdx - i) * (double)(k.table[i + 1] - k.table[i]);
     };
     const int m = std::min(k.n - 1, 8);   // slope at the kernel's end
     const double slope = ((double)k.table[k.n - 1] - (double)k.table[k.n - 1 - m]) / (m * dx);
-    double peak = 0., w0[bp::kLineDegree + 1] = {};
+    float peak = 0.f;
     for (int i = 0; i < k.n; ++i) {
         if (!std::isfinite(k.table[i])) return false;
-        peak = std::max(peak, (double)std::fabs(k.table[i]));
-    }
-    constexpr int M = 97;
-    std::vector<double> x(M), y(M), w(M);
-    for (int t = 0; t < (W + 1) / 2; ++t) {
-        const double at = t - 0.5 * (W - 1);
-        for (int i = 0; i < M; ++i) {
-            x[i] = F * std::cos(M_PI * (i + 0.5) / M);
-            const double ax = std::fabs(at - x[i]);
-            w[i] = ax <= hw ? 1. : 1e-8;
-            y[i] = ax <= hw ? weight(ax) : (double)k.table[k.n - 1] + slope * (ax - hw);
-        }
-        double c[bp::kLineDegree + 1] = {};
-        if (W % 2 == 0)
-            fit_polynomial<bp::line_degree(8)>(F, x, y, w, c);
-        else
-            fit_polynomial<bp::line_degree(9)>(F, x, y, w, c);
-        if (2 * t + 1 == W)
-            for (int d = 1; d <= bp::kLineDegree; d += 2) c[d] = 0.;   // the middle tap is even
-        auto value = [&](double f) {
-            double r = 0.;
-            for (int d = bp::kLineDegree; d >= 0; --d) r = r * f + c[d];
-            return r;
-        };
-        for (int i = 0; i <= 400; ++i) {
-            const double f = F * (i / 200. - 1.), ax = std::fabs(at - f);
-            if (ax <= hw && !(std::fabs(value(f) - weight(ax)) <= 1e-4 * peak)) return false;
-        }
-        for (int d = 0; d <= bp::kLineDegree; ++d) {
-            a->farrow[d][t] = (float)c[d];
-            if (t == 0) w0[d] = c[d];
-        }
+        peak = std::max(peak, std::fabs(k.table[i]));
     }
     // an even kernel's corrections take its weight at the end to be zero
     if (W % 2 == 0 && !(std::fabs(k.table[k.n - 1]) <= 1e-6 * peak)) return false;
-    // weights d bins past a cell's end: the tap that entered, and the
-    // continuation of the one that left
-    auto value = [&](double f) {
-        double r = 0.;
-        for (int d = bp::kLineDegree; d >= 0; --d) r = r * f + w0[d];
+    constexpr int D = Fits::D, M = Fits::kSamples, ME = Fits::kEndSamples;
+    double c[D + 1], w0[D + 1], y[M];
+    auto value = [](const double (&p)[D + 1], double f) {
+        double r = p[D];
+        for (int d = D - 1; d >= 0; --d) r = r * f + p[d];
         return r;
     };
-    const double E = 0.5 * (double)bp::kLineMaxShift;
-    constexpr int ME = 33;
-    std::vector<double> xe(ME), yi(ME), yo(ME), one(ME, 1.);
-    for (int i = 0; i < ME; ++i) {
-        xe[i] = E * std::cos(M_PI * (i + 0.5) / ME);
-        yi[i] = value(0.5 - (E + xe[i]));
-        yo[i] = value(0.5 + (E + xe[i]));
+    for (int t = 0; t < Fits::kTaps; ++t) {
+        const double at = t - 0.5 * (W - 1);
+        for (int i = 0; i < M; ++i) {
+            const double ax = std::fabs(at - fits.x[i]);
+            y[i] = ax <= hw ? weight(ax) : (double)k.table[k.n - 1] + slope * (ax - hw);
+        }
+        for (int d = 0; d <= D; ++d) {
+            const double* row = &fits.cell[t][(size_t)d * M];
+            c[d] = 0.;
+            for (int i = 0; i < M; ++i) c[d] += row[i] * y[i];
+        }
+        if (2 * t + 1 == W)
+            for (int d = 1; d <= D; d += 2) c[d] = 0.;   // the middle tap is even
+        for (int i = 0; i <= 400; ++i) {
+            const double f = Fits::F * (i / 200. - 1.), ax = std::fabs(at - f);
+            if (ax <= hw && !(std::fabs(value(c, f) - weight(ax)) <= 1e-4 * peak)) return false;
+        }
+        for (int d = 0; d <= bp::kLineDegree; ++d) {
+            a->farrow[d][t] = d <= D ? (float)c[d] : 0.f;
+            if (t == 0 && d <= D) w0[d] = c[d];
+        }
     }
-    double c[bp::kEndDegree + 1];
+    // weights d bins past a cell's end: the tap that entered, and the
+    // continuation of the one that left
     for (int s = 0; s < 2; ++s) {
-        fit_polynomial<bp::kEndDegree>(E, xe, s == 0 ? yi : yo, one, c);
+        double ce[bp::kEndDegree + 1];
+        for (int d = 0; d <= bp::kEndDegree; ++d) {
+            ce[d] = 0.;
+            for (int i = 0; i < ME; ++i) {
+                const double past = Fits::E + fits.xe[i];
+                ce[d] += fits.end[(size_t)d * ME + i] * value(w0, s == 0 ? 0.5 - past : 0.5 + past);
+            }
+        }
         // about the cell's end: substitute x - E
         double r[bp::kEndDegree + 1] = {};
         for (int d = bp::kEndDegree; d >= 0; --d) {
             for (int q = bp::kEndDegree; q >= 0; --q)
-                r[q] = (q > 0 ? r[q - 1] : 0.) - E * r[q] + (q == 0 ? c[d] : 0.);
+                r[q] = (q > 0 ? r[q - 1] : 0.) - Fits::E * r[q] + (q == 0 ? ce[d] : 0.);
         }
         for (int d = 0; d <= bp::kEndDegree; ++d) (s == 0 ? a->w_in : a->w_out)[d] = (float)r[d];
     }
     return true;
+}
+
+bool build_line_table(const bp_kernel& k, int W, bp::LineArgs* a)
+{
+    if (2.0 * k.halfwidth != (double)W) return false;
+    return W == 8 ? fit_line_table<8>(k, a) : W == 9 ? fit_line_table<9>(k, a) : false;
 }
 
 // Plain-sum table of TabulatedKernel<float> (core/Kernels.icc:137-154): entry

@@ -238,6 +238,28 @@ def test_workspace_bytes(precision, width, max_pixels, least, most):
     assert held(0) <= (9 << 20) + (1 << 20)     # 32 bytes a strip, and one strip
 
 
+@pytest.mark.parametrize("width", [8, 9])
+def test_line_plan_host_time(width):
+    """The plan of the line-interpolated sum, which every split call makes
+    before its first launch (the kernel's weight polynomials above all), takes
+    some 25 us; the least of 50 calls keeps below 100."""
+    import time
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.focus import geometry_struct
+    geometry = RadarGeometry(sim._grid(-2.5, sim.PRF, sim.R0, sim.DR, 8192, 16384),
+                             sim.straight_orbit(), core.LUT2d())
+    kernel = core.TabulatedKernelF32(core.KnabKernel(float(width), 0.8), 2048)
+    ig, kr = geometry_struct(geometry), kernel._struct()
+    times = []
+    for _ in range(50):
+        t0 = time.perf_counter()
+        n = _native.lib().bp_workspace_bytes(C.byref(ig), sim.FC, 6.0, C.byref(kr), 1,
+                                             _native.PRECISION_SPLIT, 1 << 20, 64, 1, -1)
+        times.append(time.perf_counter() - t0)
+    assert n > 0 and min(times) < 100e-6, min(times)
+
+
 def test_sincos_turns_against_long_double():
     """The plain sum's FP64 phase rotation: sin/cos of 2 pi t for t in turns
     agree with an extended-precision evaluation to a few ulp, over the
