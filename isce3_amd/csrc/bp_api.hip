@@ -1052,7 +1052,9 @@ struct LinePlan {
 // Strip height: the most lines (64, 32, 16) whose range positions stay within
 // kLineMaxShift of the middle line's at the aperture's ends, where adjacent
 // lines are P' / (fc dtau) bins apart, P' = v |p| / (|x| 2 ds prf) cycles per
-// pulse (ds = 6 m at 7.5 km/s and 1520 Hz: 0.46; 0.28 bins over 32 lines).
+// pulse (ds = 6 m at 7.5 km/s and 1520 Hz: 0.46; 0.28 bins over 32 lines).  A
+// squint adds its Doppler's part: at 400 Hz the far end has 0.44 bins, and strips
+// of 64 lines would mostly fall to the pixel-by-pixel sum.
 // Chunks of 64 pulses, of 32 where a strip's lines would turn by more than
 // the nodes interpolate within 64.
 LinePlan plan_lines(const CallArgs& a, int width, const Opts& o)
@@ -1062,6 +1064,7 @@ LinePlan plan_lines(const CallArgs& a, int width, const Opts& o)
     if (a.precision != BP_PRECISION_SPLIT || o.staged || o.lane_rows != 2 || gi.length < 1 ||
         gi.width < 32 || gi.width >= (1 << 28))
         return p;
+    double shift, dr;     // Opts::strip_shift, strip_dr
     if (!build_line_table(*a.kernel, width, &p.table)) return p;
     const bp_orbit& io = a.in_geometry->orbit;
     double vmin = INFINITY, vmax = 0., pmax = 0.;
@@ -1078,7 +1081,21 @@ LinePlan plan_lines(const CallArgs& a, int width, const Opts& o)
     const double inv_k = wvl / (2.0 * gi.range_pixel_spacing);
     const double ratio = pmax / 6.33e6;   // |p| / |x|
     if (!(vmin > 0.) || !(gi.starting_range > 0.) || !(gi.range_pixel_spacing > 0.)) return p;
-    const double shift = vmax * dt * ratio / (2.0 * a.ds) * inv_k;
+    // sine of the angle off broadside: half the aperture, the Doppler at a few
+    // points of the input grid, and what the pulses cover
+    const double half = wvl * ratio / (4.0 * a.ds);
+    double fd = 0.;
+    const bp::Lut2d dop = host_lut(a.in_geometry->doppler);
+    for (int i = 0; i < 9; ++i)
+        fd = std::max(fd, std::fabs(bp::lut2d_eval(
+                              dop, gi.sensing_start + 0.5 * (i / 3) * (gi.length - 1.) * dt,
+                              gi.starting_range + 0.5 * (i % 3) * (gi.width - 1.) * gi.range_pixel_spacing)));
+    const double squint = 0.5 * wvl * fd / vmin;
+    const double seen = squint + std::min(half, vmax * dt * gi.length / gi.starting_range);
+    const double per_sine = 2.0 * vmax / wvl * inv_k;   // bins per second between lines
+    const double shift = dt * per_sine * std::max(half, squint > 0. ? seen : 0.);
+    p.shift = per_sine * seen;
+    p.dr = gi.range_pixel_spacing;
     for (p.rows = bp::kStripLines; p.rows >= 16; p.rows /= 2)
         if (0.5 * p.rows * shift * 1.05 <= (double)bp::kLineMaxShift) break;
     if (p.rows < 16) return p;

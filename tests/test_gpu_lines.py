@@ -97,9 +97,16 @@ def test_strips_left_to_the_pixel_sum(torch_gpu, kw):
 
 
 def test_native_doppler(torch_gpu):
-    """A squinted aperture: ranges of adjacent lines are too far apart at its
-    far end, so the strips take the pixel-by-pixel sum."""
+    """A squinted aperture, whose lines lie further apart at its far end."""
     assert _run(_scene(8, doppler=400.0), 48, 64) <= 2e-4
+
+
+@pytest.mark.parametrize("doppler", [150.0, 400.0])
+@pytest.mark.parametrize("rows,cols", [(32, 64), (33, 20), (100, 70)])
+def test_squinted_strips(torch_gpu, doppler, rows, cols):
+    """The plan takes strips of 32 lines (and 32 pulses per chunk) for it, which
+    qualify: the line-interpolated sum's tolerance."""
+    assert _run(_scene(8, doppler=doppler), rows, cols) <= 6e-5
 
 
 def test_whole_and_band_by_band_agree(torch_gpu):
