@@ -786,7 +786,10 @@ struct CallArgs {
 struct Opts {
     int tile_rows, chunk, order, blocks_per_cu, lane_rows;
     bool staged;
-    int strip_rows;   // lines per strip of the line-interpolated sum, at most
+    // line-interpolated sum: lines per strip, at most; bins that two lines may lie
+    // apart per second between them; the input's range spacing
+    int strip_rows;
+    double strip_shift, strip_dr;
 };
 
 // Argument rules of focus/Backproject.cpp:77-92, the pybind binding
@@ -870,6 +873,8 @@ int check_options(const bp_options* options, Opts* o)
     if (opt.lane_rows < 0 || opt.lane_rows > 2) return fail(BP_ERR_INVALID_ARGUMENT, "lane_rows must be 0, 1 or 2");
     o->lane_rows = opt.lane_rows;  // 0: resolved by check_lane_rows
     o->strip_rows = bp::kStripLines;
+    o->strip_shift = 0.;
+    o->strip_dr = 1.;
     return BP_SUCCESS;
 }
 
@@ -903,16 +908,25 @@ int check_blocks(bp_out_block* blocks, int n_blocks, int64_t* npix)
     return BP_SUCCESS;
 }
 
-// The strips of a grid (of d.map's size): equal heights of at most max_rows
-// lines, multiples of 16 so that no wavefront tile straddles two.  Returns
-// their number.
-int64_t map_strips(bp::OutDesc& d, int max_rows)
+// The strips of a grid of d.map's size and d's spacings: equal heights of at
+// most o.strip_rows lines, multiples of 16 so that no wavefront tile straddles
+// two.  Returns their number.  None where no full strip could qualify, by
+// twice the limits: columns off the input's bins, or lines too far apart.  Such
+// grids need no fit of their strips (20 us, and four kernels of nothing).
+int64_t map_strips(bp::OutDesc& d, const Opts& o)
 {
-    const int64_t ny = (d.map.length + max_rows - 1) / max_rows;
+    const int64_t ny = (d.map.length + o.strip_rows - 1) / o.strip_rows;
     const int64_t rows = (d.map.length + ny - 1) / ny;
-    d.strip_rows = (int32_t)std::min<int64_t>(max_rows, (rows + 15) / 16 * 16);
+    d.strip_rows = (int32_t)std::min<int64_t>(o.strip_rows, (rows + 15) / 16 * 16);
     d.strips_x = (int32_t)((d.map.width + 63) / 64);
     d.strips_y = (int32_t)((d.map.length + d.strip_rows - 1) / d.strip_rows);
+    const double drift =
+        std::fabs(d.dr / o.strip_dr - 1.) * (double)(std::min<int64_t>(d.map.width, 64) - 1);
+    const double apart = 0.5 * std::min<int64_t>(d.map.length, d.strip_rows) * d.dt * o.strip_shift;
+    if (drift > 2. * (double)bp::kLineColumnTol || apart > 2. * (double)bp::kLineMaxShift) {
+        d.strips_x = d.strips_y = 0;
+        d.strip_info = -1;
+    }
     return (int64_t)d.strips_x * d.strips_y;
 }
 
@@ -925,7 +939,7 @@ int plan_batch(const bp_out_block* blocks, int n_blocks, const Opts& o, int32_t*
     block_of_grid.clear();
     auto* descs = reinterpret_cast<bp::OutDesc*>(dst + sizeof(bp::BatchHeader));
     int64_t n_seq = 0, n_rec = 0, n_strips = 0;
-    int g = 0;
+    int g = 0, no_strips = 0;
     for (int b = 0; b < n_blocks; ++b) {
         const bp_grid& go = blocks[b].grid;
         if (go.length * go.width == 0) continue;
@@ -945,7 +959,9 @@ int plan_batch(const bp_out_block* blocks, int n_blocks, const Opts& o, int32_t*
         d.failed = d_failed + g;
         d.strip_seq = n_strips;
         d.strip_info = n_strips;
-        n_strips += map_strips(d, o.strip_rows);
+        const int64_t strips = map_strips(d, o);
+        if (strips == 0) no_strips = 1;
+        n_strips += strips;
         n_seq += d.map.n_tiles;
         n_rec += go.length * go.width;
         std::memcpy(descs + g, &d, sizeof(d));
@@ -959,6 +975,7 @@ int plan_batch(const bp_out_block* blocks, int n_blocks, const Opts& o, int32_t*
     hdr->n_grids = g;
     hdr->lane_rows = o.lane_rows;
     hdr->n_strips = n_strips;
+    hdr->no_strips = no_strips;
     if (hdr->n_geom_groups > INT32_MAX / 2) return fail(BP_ERR_INVALID_ARGUMENT, "too many output pixels");
     std::memcpy(dst, hdr, sizeof(*hdr));
     return BP_SUCCESS;
@@ -1045,6 +1062,7 @@ struct Step {
 struct LinePlan {
     bool on;
     int rows, chunk_log2, slots;
+    double shift, dr;     // Opts::strip_shift, strip_dr
     size_t strip_bytes;
     bp::LineArgs table;   // the weight polynomials
 };
@@ -1064,7 +1082,6 @@ LinePlan plan_lines(const CallArgs& a, int width, const Opts& o)
     if (a.precision != BP_PRECISION_SPLIT || o.staged || o.lane_rows != 2 || gi.length < 1 ||
         gi.width < 32 || gi.width >= (1 << 28))
         return p;
-    double shift, dr;     // Opts::strip_shift, strip_dr
     if (!build_line_table(*a.kernel, width, &p.table)) return p;
     const bp_orbit& io = a.in_geometry->orbit;
     double vmin = INFINITY, vmax = 0., pmax = 0.;
@@ -1110,6 +1127,14 @@ LinePlan plan_lines(const CallArgs& a, int width, const Opts& o)
     p.strip_bytes = bp::line_strip_bytes(p.slots, p.table.n_sums);
     p.on = p.strip_bytes <= kStripBytes;
     return p;
+}
+
+void use_plan(Opts& o, const LinePlan& p)
+{
+    if (!p.on) return;
+    o.strip_rows = p.rows;
+    o.strip_shift = p.shift;
+    o.strip_dr = p.dr;
 }
 
 // Segments of the plain sum that get wavefronts of their own (0: none).  The
@@ -1420,7 +1445,7 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
     if (npix > 0 && gi.length * gi.width > 0 && a.in_dev == nullptr)
         return fail(BP_ERR_INVALID_ARGUMENT, "in is null");
     LinePlan lp = plan_lines(a, width, o);
-    if (lp.on) o.strip_rows = lp.rows;
+    use_plan(o, lp);
     StaticData fixed_st;
     Scratch fixed_sc;
     if (carve && (rc = carve_call(*carve, a, width, n_blocks, npix, fixed_st, fixed_sc)) != BP_SUCCESS)
@@ -1454,7 +1479,7 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
     if (a.precision == BP_PRECISION_SPLIT && (rc = ensure(sc.split, sizeof(bp::PixSplit) * n_rec)))
         return rc;
     int64_t group = 0;
-    if (lp.on) {
+    if (lp.on && hdr.n_strips > 0) {
         if (carve) {
             group = carve_lines(*carve, lp, hdr.n_strips, sc);
         } else {
@@ -1683,7 +1708,7 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
         return fail(BP_ERR_INVALID_ARGUMENT, "in is null");
     if (npix == 0) return BP_SUCCESS;
     const LinePlan lp = plan_lines(a, width, o);
-    if (lp.on) o.strip_rows = lp.rows;
+    use_plan(o, lp);
 
     BP_HIP_CHECK(hipSetDevice(c->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1719,7 +1744,7 @@ int run_host(bp_context* c, const CallArgs& a, bp_out_block* blk, int64_t batch,
     if (a.precision == BP_PRECISION_SPLIT && (rc = ensure(c->sc.split, sizeof(bp::PixSplit) * npix)))
         return rc;
     const int64_t group =
-        lp.on ? alloc_lines(lp, hdr.n_strips, hdr.n_strips, c->workspace_limit, c->sc) : 0;
+        lp.on && hdr.n_strips > 0 ? alloc_lines(lp, hdr.n_strips, hdr.n_strips, c->workspace_limit, c->sc) : 0;
     BP_HIP_CHECK(bp::launch_clear(static_cast<int32_t*>(c->sc.flags.ptr), n_flag, s));
     if ((rc = pulse_states(c->st, a, static_cast<int32_t*>(c->sc.flags.ptr), s))) return rc;
 
@@ -2385,15 +2410,18 @@ try {
     // strips in groups of the scene's workspace; graphs for powers of two of them
     int64_t groups = 0;
     if (sc->lines.on && o.lane_rows == 2 && !o.staged) {
-        o.strip_rows = sc->lines.rows;
+        use_plan(o, sc->lines);
         int64_t n_strips = 0;
         for (int b = 0; b < n_blocks; ++b) {
             bp::OutDesc d;
             d.map.length = blocks[b].grid.length;
             d.map.width = blocks[b].grid.width;
-            if (d.map.length * d.map.width > 0) n_strips += map_strips(d, o.strip_rows);
+            d.dt = 1.0 / blocks[b].grid.prf;
+            d.dr = blocks[b].grid.range_pixel_spacing;
+            if (d.map.length * d.map.width > 0) n_strips += map_strips(d, o);
         }
-        for (groups = 1; groups * sc->line_group < n_strips;) groups *= 2;
+        if (n_strips > 0)
+            for (groups = 1; groups * sc->line_group < n_strips;) groups *= 2;
     }
 
     bp_scene::Graph* g = nullptr;

@@ -147,7 +147,8 @@ struct OutDesc {
     float2* out;                // complex64 [length x width]
     float* height;              // optional float32 [length x width]
     int32_t* failed;            // per-grid flag: some pixel failed to converge
-    // strips of the line-interpolated split sum: strip_rows x 64 pixels, row
+    // strips of the line-interpolated split sum (none: strip_info < 0): strip_rows
+    // x 64 pixels, row
     // (y, x) of strips with its StripInfo at strip_info + y strips_x + x; the
     // batch's strips are numbered consecutively, column by column in a grid
     int32_t strip_rows, strips_x, strips_y, pad2_;
@@ -167,7 +168,7 @@ struct BatchHeader {
     int64_t n_strips;           // strips of all grids
     int32_t plain_segs;         // plain sum: segments summed by their own
                                 // wavefronts, 0: each wavefront takes them all
-    int32_t pad_;
+    int32_t no_strips;          // some grid has none
 };
 static_assert(sizeof(BatchHeader) == 48, "BatchHeader layout");
 

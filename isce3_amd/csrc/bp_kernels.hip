@@ -274,6 +274,7 @@ __device__ inline PixSplit fit_pixel(const GeomArgs& a, const PixGeom& g, bool h
 __device__ inline bool strip_skipped(const StripInfo* strips, int pass, const OutDesc& d,
                                      int64_t tile)
 {
+    if (d.strip_info < 0) return !(pass & kPassLeft);
     const int64_t ty = tile / d.map.tiles_x, tx = tile - ty * d.map.tiles_x;
     const int64_t y = ty * d.map.tile_rows * d.map.lane_rows / d.strip_rows;
     const int64_t x = tx * d.map.tile_cols / 64;
@@ -281,10 +282,11 @@ __device__ inline bool strip_skipped(const StripInfo* strips, int pass, const Ou
     return !((ok == kStripLeft && (pass & kPassLeft)) || (ok == kStripRedo && (pass & kPassRedo)));
 }
 
-// Whether such a launch has no strip at all.
-__device__ inline bool pass_empty(const int32_t* n_left, int pass)
+// Whether such a launch has no tile at all.
+__device__ inline bool pass_empty(const BatchHeader* batch, const int32_t* n_left, int pass)
 {
-    const int n = ((pass & kPassLeft) ? n_left[0] : 0) + ((pass & kPassRedo) ? n_left[1] : 0);
+    const int n = ((pass & kPassLeft) ? n_left[0] + batch->no_strips : 0) +
+                  ((pass & kPassRedo) ? n_left[1] : 0);
     return __builtin_amdgcn_readfirstlane(n) == 0;
 }
 
@@ -368,7 +370,7 @@ void fit_kernel(GeomArgs a)
 {
     const int64_t ng = uniform64(a.batch->n_groups);
     if ((int64_t)blockIdx.x >= ng) return;
-    if (a.strips != nullptr && pass_empty(a.flags + 2, a.strip_pass)) return;
+    if (a.strips != nullptr && pass_empty(a.batch, a.flags + 2, a.strip_pass)) return;
     const OutDesc* grids = batch_grids(a.batch);
     const int n_grids = __builtin_amdgcn_readfirstlane(a.batch->n_grids);
     const int64_t n_seq = uniform64(a.batch->n_seq);
@@ -1454,7 +1456,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 void sum_split_kernel(SumArgs a)
 {
     static_assert(!(kPair && kStaged), "two-line lanes gather their taps");
-    if (a.strips != nullptr && pass_empty(a.n_left, a.strip_pass)) return;
+    if (a.strips != nullptr && pass_empty(a.batch, a.n_left, a.strip_pass)) return;
     constexpr int ROW = poly_row_floats(W);
     constexpr int kTable = kPair ? PairTable<W>::kFloats : (kPolyphaseRows + 1) * ROW;
     // static LDS arrays: row and slot offsets fold into the ds_read offsets

@@ -109,6 +109,63 @@ def test_squinted_strips(torch_gpu, doppler, rows, cols):
     assert _run(_scene(8, doppler=doppler), rows, cols) <= 6e-5
 
 
+def test_grids_without_strips(torch_gpu):
+    """Grids off the input's range spacing, or with lines too far apart, beside
+    one of strips in a batch: each as alone, to the bit, and alone they take no
+    strip workspace."""
+    import ctypes as C
+    from isce3_amd import _native, sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import LUT2d
+    from isce3_amd.focus import backproject, backproject_blocks
+    orb, in_geom, dem, raw, kernel = _scene(8)
+    d_raw = torch_gpu.from_numpy(raw).to("cuda:0")
+
+    def grid(rows, cols, dr=1.0, prf=1.0):
+        return sim._grid(-0.5 * rows / sim.PRF, sim.PRF / prf, sim.R0 + 40 * sim.DR, dr * sim.DR,
+                         rows, cols)
+
+    grids = [grid(64, 70, dr=0.75), grid(65, 70), grid(48, 70, prf=5.0), grid(33, 64),
+             grid(20, 40, dr=1.25)]
+    geoms = [RadarGeometry(g, orb, LUT2d()) for g in grids]
+
+    def empty(g):
+        return torch_gpu.empty(tuple(g.shape), dtype=torch_gpu.complex64, device="cuda:0")
+
+    alone = [empty(g) for g in grids]
+    for o, g in zip(alone, geoms):
+        backproject(o, g, d_raw, in_geom, dem, sim.FC, 6.0, kernel, "nodelay", precision="split")
+    batch = [empty(g) for g in grids]
+    backproject_blocks(batch, geoms, d_raw, in_geom, dem, sim.FC, 6.0, kernel, "nodelay",
+                       precision="split")
+    for a, b in zip(alone, batch):
+        np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
+
+    def taken(g):
+        from isce3_amd.focus import geometry_struct, parse_geo2rdr_params, parse_rdr2geo_params
+        ctx, st, failed = C.c_void_p(), _native.Stats_t(), C.c_int(0)
+        lib = _native.lib()
+        _native.check(lib.bp_context_create(0, C.byref(ctx)))
+        out, geom = empty(g), RadarGeometry(g, orb, LUT2d())
+        og, ig = geometry_struct(geom), geometry_struct(in_geom)
+        dm, kr, opt = dem._struct(), kernel._struct(), _native.Options_t()
+        r2g, g2r = parse_rdr2geo_params({}), parse_geo2rdr_params({})
+        torch_gpu.cuda.synchronize()
+        free = torch_gpu.cuda.mem_get_info(0)[0]
+        rc = lib.bp_backproject(ctx, C.byref(og), C.byref(ig), C.byref(dm), sim.FC, 6.0, C.byref(kr),
+                                0, C.byref(r2g), C.byref(g2r), C.c_void_p(d_raw.data_ptr()),
+                                C.c_void_p(out.data_ptr()), None, _native.PRECISION_SPLIT,
+                                C.byref(opt), None, C.byref(failed), C.byref(st))
+        n = free - torch_gpu.cuda.mem_get_info(0)[0]
+        _native.check(rc)
+        lib.bp_context_destroy(ctx)
+        return n
+
+    # 4096 pixels of 112 bytes a strip, against 0.3 MB of workspace as well
+    assert taken(grid(640, 640, dr=0.75)) <= 640 * 640 * 112 + (8 << 20)
+    assert taken(grid(640, 640)) >= 640 * 640 * 112 + (24 << 20)
+
+
 def test_whole_and_band_by_band_agree(torch_gpu):
     """Pulses in host memory under a budget below a strip's window: the strip's
     pulses go through the device in parts, with the same result to the bit."""
