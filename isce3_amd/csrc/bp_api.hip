@@ -136,6 +136,27 @@ struct HostPath {
     std::vector<hipEvent_t> timing;               // per band: copy start/end, sum start/end
 };
 
+// A second stream for the strips that the line-interpolated sum leaves, and the
+// events that part it from the call's stream and join it again.
+struct Branch {
+    hipStream_t s = nullptr;   // default priority
+    hipEvent_t part = nullptr, fit = nullptr, join = nullptr;
+    bool create()
+    {
+        return hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess &&
+               hipEventCreateWithFlags(&part, hipEventDisableTiming) == hipSuccess &&
+               hipEventCreateWithFlags(&fit, hipEventDisableTiming) == hipSuccess &&
+               hipEventCreateWithFlags(&join, hipEventDisableTiming) == hipSuccess;
+    }
+    void destroy()
+    {
+        if (part) (void)hipEventDestroy(part);
+        if (fit) (void)hipEventDestroy(fit);
+        if (join) (void)hipEventDestroy(join);
+        if (s) (void)hipStreamDestroy(s);
+    }
+};
+
 struct bp_context {
     int device = 0;
     int n_cu = 0;
@@ -146,6 +167,7 @@ struct bp_context {
     Scratch sc;
     HostPath hp;
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
+    Branch branch;
     std::vector<unsigned char> desc_host;
     std::vector<int> desc_block;
     std::vector<int32_t> flags_host;
@@ -676,13 +698,14 @@ try {
     if (hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
         c->n_cu < 1)
         c->n_cu = 256;
-    for (auto& ev : c->ev) {
-        if (hipEventCreate(&ev) != hipSuccess) {
-            for (auto& e2 : c->ev)
-                if (e2) (void)hipEventDestroy(e2);
-            delete c;
-            return fail(BP_ERR_HIP, "hipEventCreate failed");
-        }
+    bool made = c->branch.create();
+    for (auto& ev : c->ev) made = made && hipEventCreate(&ev) == hipSuccess;
+    if (!made) {
+        c->branch.destroy();
+        for (auto& ev : c->ev)
+            if (ev) (void)hipEventDestroy(ev);
+        delete c;
+        return fail(BP_ERR_HIP, "hipEventCreate failed");
     }
     // a failed lookup disables bp_backproject_noalloc only
     if (scratch_address(device, &c->scratch) != BP_SUCCESS) {
@@ -749,6 +772,7 @@ try {
     free_static(c->st);
     free_scratch(c->sc);
     free_host_path(c->hp);
+    c->branch.destroy();
     for (auto& ev : c->ev)
         if (ev) (void)hipEventDestroy(ev);
     delete c;
@@ -1051,6 +1075,7 @@ struct Step {
     // line-interpolated sum (split; lines false: every pixel at every pulse)
     int segs;              // plain: segments with wavefronts of their own
     bool lines;
+    const Branch* branch;  // lines: strips that are left run beside them, or null
     bp::LineArgs la;
     int64_t n_strips;      // of the batch (the fit's grid)
     int64_t group_strips;  // strips the workspace holds
@@ -1303,6 +1328,7 @@ void build_step(Step& sp, const StaticData& st, const Scratch& sc, const CallArg
     sp.flag_words = 0;
     sp.ev[0] = sp.ev[1] = sp.ev[2] = nullptr;
     sp.lines = false;
+    sp.branch = nullptr;
     sp.segs = 0;
 }
 
@@ -1346,10 +1372,30 @@ int enqueue_sum(const Step& sp, const bp::BatchHeader* batch, const float2* rc, 
     bp::SumArgs sa = sp.sa;
     sa.batch = batch;
     sa.rc = rc;
+    bp::GeomArgs ga = sp.ga;
+    ga.batch = batch;
     if (sp.lines) {
-        // the strips in groups of the workspace's size, then the strips that
-        // did not qualify or met samples that are not finite: their pixels'
-        // records are fitted only now
+        // The strips in groups of the workspace's size; beside them the strips
+        // that did not qualify, whose pixels walk their aperture alone (1.4 ms
+        // however few they are: behind the line sum a tile of 310 x 290 pixels with
+        // a column of such strips took 4.80 ms, with none of its strips taken 4.46);
+        // then those that met samples that are not finite.  The strips wait for the
+        // other stream's fit, so that its sum, next there, has its long wavefronts
+        // placed first, evenly over the SIMDs: 512 x 512 pixels of which most strips
+        // are left 7.9 ms when the line sum came first, 5.0 so.
+        ga.strip_pass = sa.strip_pass = bp::kPassLeft | bp::kPassRedo;
+        if (sp.branch) {
+            ga.strip_pass = sa.strip_pass = bp::kPassLeft;
+            const hipStream_t o = sp.branch->s;
+            BP_HIP_CHECK(hipEventRecord(sp.branch->part, s));
+            BP_HIP_CHECK(hipStreamWaitEvent(o, sp.branch->part, 0));
+            BP_HIP_CHECK(bp::launch_fit(ga, groups, o));
+            BP_HIP_CHECK(hipEventRecord(sp.branch->fit, o));
+            BP_HIP_CHECK(bp::launch_sum_split(sa, sp.width, sp.sum_grid, sp.staged, sp.pair, o));
+            BP_HIP_CHECK(hipEventRecord(sp.branch->join, o));
+            BP_HIP_CHECK(hipStreamWaitEvent(s, sp.branch->fit, 0));
+            ga.strip_pass = sa.strip_pass = bp::kPassRedo;
+        }
         bp::LineArgs la = sp.la;
         la.batch = batch;
         la.rc = rc;
@@ -1359,8 +1405,7 @@ int enqueue_sum(const Step& sp, const bp::BatchHeader* batch, const float2* rc, 
             la.s_end = s0 + n;
             BP_HIP_CHECK(bp::launch_strips(la, sp.width, true, s));
         }
-        bp::GeomArgs ga = sp.ga;
-        ga.batch = batch;
+        if (sp.branch) BP_HIP_CHECK(hipStreamWaitEvent(s, sp.branch->join, 0));
         BP_HIP_CHECK(bp::launch_fit(ga, groups, s));
     }
     if (sp.precision == BP_PRECISION_PLAIN)
@@ -1491,7 +1536,10 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
 
     Step sp;
     build_step(sp, st, sc, a, width, o, c->n_cu);
-    if (group > 0) set_lines(sp, lp, sc, a, hdr.n_strips, group);
+    if (group > 0) {
+        set_lines(sp, lp, sc, a, hdr.n_strips, group);
+        sp.branch = &c->branch;
+    }
     if (segs > 0) {
         sp.segs = segs;
         sp.sa.parts = static_cast<double2*>(sc.parts.ptr);
@@ -1501,7 +1549,10 @@ int run_blocks(bp_context* c, const CallArgs& a, bp_out_block* blocks, int n_blo
     sp.flag_words = 0;  // cleared above, before the pulse states
     if (stats)
         for (int i = 0; i < 3; ++i) sp.ev[i] = c->ev[i];
-    if ((rc = enqueue_step(sp, (int)hdr.n_groups, s))) return rc;
+    if ((rc = enqueue_step(sp, (int)hdr.n_groups, s))) {
+        (void)hipStreamSynchronize(c->branch.s);   // nothing of the call runs on
+        return rc;
+    }
 
     c->flags_host.assign(n_flag, 0);
     BP_HIP_CHECK(hipMemcpyAsync(c->flags_host.data(), sc.flags.ptr, sizeof(int32_t) * n_flag,
@@ -2120,6 +2171,14 @@ struct bp_scene {
     unsigned char* h_desc = nullptr;   // pinned: header + max_blocks descriptors
     int32_t* h_flags = nullptr;        // pinned: kFlagWords + max_blocks words
     hipStream_t cap = nullptr;         // capture stream (default priority)
+    Branch branch;
+    // Strips were left by the last batch: the next one is launched kernel by kernel,
+    // with the strips that are left beside the others.  In a graph the second branch
+    // takes 17 us (one strip) to 44 us (25) longer to replay, and its long wavefronts
+    // share SIMDs where the line sum's are placed first (512 x 512 pixels with a
+    // column of such strips: 7.4 ms instead of 4.8); a graph without it puts 0.3 ms of
+    // line sum before them.  Results are the same either way.
+    bool left = false;
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     std::vector<int> block_of_grid;
     LinePlan lines{};          // line-interpolated sum (lane_rows 2)
@@ -2169,6 +2228,7 @@ void destroy_scene(bp_scene* sc)
     for (auto& ev : sc->ev)
         if (ev) (void)hipEventDestroy(ev);
     if (sc->cap) (void)hipStreamDestroy(sc->cap);
+    sc->branch.destroy();
     delete sc;
 }
 
@@ -2280,6 +2340,25 @@ int capture_graph(bp_scene* sc, const Opts& o, int64_t groups, bp_scene::Graph* 
     return BP_SUCCESS;
 }
 
+// The step of a batch launched kernel by kernel.
+int launch_scene(bp_scene* sc, const Opts& o, const bp::BatchHeader& hdr, hipStream_t s)
+{
+    Step sp;
+    build_step(sp, sc->st, sc->sc, sc->args, sc->width, o, sc->ctx->n_cu);
+    set_lines(sp, sc->lines, sc->sc, sc->args, hdr.n_strips, sc->line_group);
+    sp.branch = &sc->branch;
+    sp.geom_grid = (int)hdr.n_geom_groups;
+    sp.flag_words = kFlagWords + sc->max_blocks;
+    BP_HIP_CHECK(hipMemcpyAsync(sc->sc.desc.ptr, sc->h_desc,
+                                sizeof(bp::BatchHeader) + sizeof(bp::OutDesc) * hdr.n_grids,
+                                hipMemcpyHostToDevice, s));
+    const int rc = enqueue_step(sp, (int)hdr.n_groups, s);
+    if (rc != BP_SUCCESS) return rc;
+    BP_HIP_CHECK(hipMemcpyAsync(sc->h_flags, sc->sc.flags.ptr, sizeof(int32_t) * sp.flag_words,
+                                hipMemcpyDeviceToHost, s));
+    return BP_SUCCESS;
+}
+
 }  // namespace
 
 extern "C" {
@@ -2321,7 +2400,7 @@ try {
         destroy_scene(sc);
         return code;
     };
-    if (hipStreamCreateWithFlags(&sc->cap, hipStreamNonBlocking) != hipSuccess)
+    if (hipStreamCreateWithFlags(&sc->cap, hipStreamNonBlocking) != hipSuccess || !sc->branch.create())
         return bail(fail(BP_ERR_HIP, "hipStreamCreate failed"));
     for (auto& ev : sc->ev)
         if (hipEventCreate(&ev) != hipSuccess) return bail(fail(BP_ERR_HIP, "hipEventCreate failed"));
@@ -2424,12 +2503,13 @@ try {
             for (groups = 1; groups * sc->line_group < n_strips;) groups *= 2;
     }
 
+    const bool replayed = groups == 0 || !sc->left;
     bp_scene::Graph* g = nullptr;
     for (auto& x : sc->graphs)
         if (x.chunk == o.chunk && x.blocks_per_cu == o.blocks_per_cu && x.staged == o.staged &&
             x.lane_rows == o.lane_rows && x.groups == groups)
             g = &x;
-    if (g == nullptr) {
+    if (g == nullptr && replayed) {
         bp_scene::Graph ng{};
         if ((rc = capture_graph(sc, o, groups, &ng)) != BP_SUCCESS) return rc;
         sc->graphs.push_back(ng);
@@ -2445,7 +2525,8 @@ try {
         hdr.plain_segs = plain_segments(sc->args, hdr.n_seq, npix, -1);
         std::memcpy(sc->h_desc, &hdr, sizeof(hdr));
     }
-    for (const bp_scene::GridNode& gn : g->nodes) {
+    for (size_t i = 0; replayed && i < g->nodes.size(); ++i) {
+        const bp_scene::GridNode& gn = g->nodes[i];
         const int64_t n = std::min(std::max<int64_t>(hdr.n_strips - gn.first, 0), gn.count);
         int64_t grid;
         switch (gn.kind) {
@@ -2460,9 +2541,17 @@ try {
         BP_HIP_CHECK(hipGraphExecKernelNodeSetParams(g->exec, gn.node, &p));
     }
     if (stats) BP_HIP_CHECK(hipEventRecord(sc->ev[0], s));
-    BP_HIP_CHECK(hipGraphLaunch(g->exec, s));
+    if (replayed) {
+        BP_HIP_CHECK(hipGraphLaunch(g->exec, s));
+    } else if ((rc = launch_scene(sc, o, hdr, s)) != BP_SUCCESS) {
+        (void)hipStreamSynchronize(sc->branch.s);   // nothing of the call runs on
+        (void)hipStreamSynchronize(s);
+        return rc;
+    }
     if (stats) BP_HIP_CHECK(hipEventRecord(sc->ev[2], s));
     BP_HIP_CHECK(hipStreamSynchronize(s));
+    if (groups > 0)
+        sc->left = sc->h_flags[2] + hdr.no_strips > 0 && sc->h_flags[2] < hdr.n_strips;
     const hipEvent_t ev[3] = {sc->ev[0], nullptr, sc->ev[2]};
     return finish_step(sc->h_flags, hdr.n_grids, sc->block_of_grid, blocks, ev, any_failed, stats);
 } catch (...) {

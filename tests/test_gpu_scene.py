@@ -144,6 +144,35 @@ def test_strip_counts_without_allocation(torch_gpu):
         assert taken <= 16 << 20
 
 
+def test_strips_left_beside_others(torch_gpu):
+    """Blocks at the swath's edge, where some strips are left to the pixel-by-pixel
+    sum: replayed, and launched beside the others once the scene has met such strips;
+    then blocks without any, all as eager."""
+    from isce3_amd import sim
+    from isce3_amd.focus import Scene
+    torch = torch_gpu
+    sc = sim.make_scene("tiny")
+    na, nr = 1600, 400
+    sc.in_grid = sim._grid(-0.5 * na / sim.PRF, sim.PRF, sim.R0, sim.DR, na, nr)
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(6)
+    raw_dev = torch.randn((na, nr), dtype=torch.complex64, device="cuda:0", generator=gen)
+
+    def block(rows, cols, c0, dr=1.0):
+        return sim._grid(-0.5 * rows / sim.PRF, sim.PRF, sim.R0 + c0 * sim.DR, dr * sim.DR, rows, cols)
+
+    edge = [block(100, 170, -20), block(33, 64, 100), block(40, 50, 150, 0.7)]
+    inside = [block(70, 100, 100)]
+    with Scene(raw_dev, sc.in_geometry(), sc.orbit, sc.doppler, sc.dem, sc.fc, sc.ds, sc.kernel,
+               sc.dry_tropo_model, precision="split", max_pixels=1 << 15, max_blocks=4) as scene:
+        for b in (edge, edge, edge, inside, inside, edge):
+            ref = eager(sc, raw_dev, b, "split", {})
+            outs, _, _, st = replay(scene, b, {}, heights=False)
+            for z, z0 in zip(outs, ref[0]):
+                np.testing.assert_array_equal(z, z0)
+            assert st["updates"] == ref[3]["updates"]
+
+
 @pytest.mark.parametrize("precision,limit", [("split", -1), ("split", 20 << 20), ("plain", -1)])
 def test_memory_held_as_stated(torch_gpu, precision, limit):
     """A scene takes at most its per-pixel scratch and bp_workspace_bytes (and
