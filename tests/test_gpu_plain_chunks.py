@@ -84,3 +84,35 @@ def test_segments_and_whole_windows_agree(torch_gpu):
                     DEMInterpolator(50.0), sim.FC, 40.0, kernel, "nodelay", precision="plain")
         outs.append(out)
     np.testing.assert_array_equal(outs[0][:33], outs[1])
+
+
+def test_chunk_phase_against_single_delays(torch_gpu):
+    """63 pulses as the first of a whole chunk (delays by the cubic, the pulses
+    behind them zero) and as a chunk that the data's end cuts off (a delay per
+    pulse), at a wavelength of 2.4 mm: 7e8 cycles, so that FP64 rounding shows.
+    What is left between the two is the rounding of a delay per pulse, five
+    roundings of half an ulp of 7e8 cycles (7.5e-7 rad each at most, 2.2e-7 RMS):
+    4.8e-7; the cubic of delays in two words adds less than 2e-7 to it, rounded
+    delays at its nodes would add as much again (6.6e-7 was measured)."""
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import KnabKernel, LUT2d, TabulatedKernelF32
+    from isce3_amd.focus import backproject
+    from isce3_amd.geometry import DEMInterpolator
+    nr, rows, cols = 96, 40, 40
+    orb = sim.straight_orbit()
+    og = RadarGeometry(sim._grid(-0.5 * rows / sim.PRF, sim.PRF, sim.R0 + 12.3 * sim.DR, sim.DR,
+                                 rows, cols), orb, LUT2d())
+    rng = np.random.default_rng(2)
+    raw = np.zeros((127, nr), np.complex64)
+    raw[:63] = rng.standard_normal((63, nr)) + 1j * rng.standard_normal((63, nr))
+    outs = []
+    for na in (127, 63):
+        ig = RadarGeometry(sim._grid(-32 / sim.PRF, sim.PRF, sim.R0, sim.DR, na, nr), orb, LUT2d())
+        out = np.empty((rows, cols), np.complex64)
+        backproject(out, og, raw[:na], ig, DEMInterpolator(50.0), 100 * sim.FC, 0.01,
+                    TabulatedKernelF32(KnabKernel(8.0, 0.8), 2048), "nodelay", precision="plain")
+        outs.append(out.astype(complex))
+    rel = np.linalg.norm(outs[0] - outs[1]) / np.linalg.norm(outs[1])
+    print(f"[plain chunks] cubic and single delays differ by {rel:.2e}", flush=True)
+    assert rel <= 5.2e-7
