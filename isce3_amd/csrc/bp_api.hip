@@ -1048,6 +1048,28 @@ int upload_static(StaticData& st, const CallArgs& a, int width, hipStream_t s)
 }
 
 // Platform position/velocity at every pulse (plain precision).
+// Whether the plain sum's chunks are worth their nodes: a pixel at the swath's
+// near edge keeps the cubic's tolerance.  The cubic is off
+// by the fourth derivative of the phase, at most 3 v^4 / R^3 of range in a straight
+// pass, times 5,666 pulses^4 (the nodes' polynomial over 4!); the third difference
+// is at most 0.86 v^3 / R^2 of range.  At 5 km, 120 m/s and L band that holds from
+// a PRF of 700 Hz on; at 100 Hz, where no chunk keeps the tolerance, trying cost 28 %.
+bool plain_chunks(const CallArgs& a)
+{
+    const bp_grid& gi = a.in_geometry->grid;
+    const bp_orbit& io = a.in_geometry->orbit;
+    double v2 = 0.;
+    for (int i = 0; i < io.n; ++i)
+        v2 = std::max(v2, io.vel[3 * i] * io.vel[3 * i] + io.vel[3 * i + 1] * io.vel[3 * i + 1] +
+                              io.vel[3 * i + 2] * io.vel[3 * i + 2]);
+    const double r = gi.starting_range, step = std::sqrt(v2) / gi.prf;   // metres per pulse
+    const double per_metre = 2. * a.fc / bp::kC;
+    const double off = per_metre * 5666. * 3. * step * step * step * step / (r * r * r);
+    const double eps = 2. * M_PI * per_metre * 0.86 * step * step * step / (r * r);
+    return r > 0. && off <= std::max(bp::kCubicTol, bp::kCubicUlps * per_metre * r) &&
+           eps <= bp::kCubicEps;
+}
+
 int pulse_states(StaticData& st, const CallArgs& a, int32_t* d_flags, hipStream_t s)
 {
     if (a.precision != BP_PRECISION_PLAIN) return BP_SUCCESS;
@@ -1315,6 +1337,7 @@ void build_step(Step& sp, const StaticData& st, const Scratch& sc, const CallArg
     sa.inv_dtau = 1.0 / dtau;
     sa.exact_width = 2.0 * a.kernel->halfwidth == (double)width;
     sa.tab2 = static_cast<const double2*>(st.table2.ptr);
+    sa.chunks = a.precision == BP_PRECISION_PLAIN && plain_chunks(a);
 
     sp.width = width;
     sp.precision = a.precision;
@@ -2288,7 +2311,7 @@ int capture_graph(bp_scene* sc, const Opts& o, int64_t groups, bp_scene::Graph* 
     const void* geo_fn = bp::kernel_fn(bp::dem_generic(host_dem(sc->dem)) ? 4 : 0, sc->width,
                                        o.staged, pair);
     const bool plain = sc->args.precision == BP_PRECISION_PLAIN;
-    const void* tile_fn = bp::kernel_fn(plain ? 1 : 3, sc->width, o.staged, pair);
+    const void* tile_fn = bp::kernel_fn(plain ? (sp.sa.chunks ? 1 : 6) : 3, sc->width, o.staged, pair);
     const void* total_fn = plain && sc->part_records > 0 ? bp::kernel_fn(5, sc->width, false, false)
                                                          : nullptr;
     for (hipGraphNode_t nd : nodes) {

@@ -134,6 +134,15 @@ constexpr int kPlainNode[4] = {2, 19, 44, 61};
 // not fit (2.4e-7 m) or that the data's end cuts off: delays are evaluated there.
 constexpr double kPosQ = 4398046511104.0;  // 2^42
 constexpr unsigned long long kPosNone = 1ull << 63;
+// How far the cubic may be off the delay (cycles): a few roundings of the phase
+// itself, 8 / 2^53 of fc tau (4e-8 rad at 850 km and L band), and no less than
+// 6e-9 rad.
+constexpr double kCubicUlps = 8. / 9007199254740992.;
+constexpr double kCubicTol = 1e-9;
+// Largest third difference of the phase (radians), whose phasor 1 + i eps is
+// good to 2e-8 at the chunk's end (eps^2 / 2 times 64^3 / 6); 7e-9 at 850 km, 7.5
+// km/s, 1520 Hz and L band, and beyond 2e-7 only where the phase rounds to more.
+constexpr double kCubicEps = 9e-7;
 
 // One output grid of a (batched) call.  Wavefront tiles of all grids are
 // numbered consecutively: grid g owns [seq_base, seq_base + map.n_tiles).
@@ -321,6 +330,7 @@ struct SumArgs {
     int32_t strip_pass;         // StripPass bits of this launch
     double2* parts;             // plain: segment sums [segment][record], or null
     int64_t parts_stride;       // records per segment
+    int32_t chunks;             // plain: delays by chunks of pulses (the kernel's choice)
 };
 
 // Host launchers (defined in bp_kernels.hip).  `grid` is the number of
@@ -356,7 +366,7 @@ hipError_t launch_strips(const LineArgs& a, int width, bool last, hipStream_t st
 hipError_t launch_band_window(const PixGeom* geom, int64_t length, int64_t width, int band_rows,
                               int64_t n_bands, int32_t* win, hipStream_t stream);
 // Host-side handle of a kernel (0 geometry, 4 geometry for generic DEMs,
-// 1 plain sum, 5 its segments' total, 2 split sum, 3 fit),
+// 1 plain sum, 6 with a delay per pulse, 5 its segments' total, 2 split sum, 3 fit),
 // as graph kernel nodes report it.
 const void* kernel_fn(int which, int width, bool staged, bool pair);
 

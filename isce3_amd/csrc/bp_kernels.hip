@@ -67,7 +67,7 @@ __device__ inline double newton3_at(const Newton3& c, double j)
 // its four delays to all of its pulses, where they no longer average out over the
 // chunk: 5.8e-9 rad RMS in a chunk's mean phase with plain delays (2.7e-9 with a delay
 // per pulse), 1.9e-9 so.  Error of a 256 x 256 chip, RMS of eight: 8.46e-8 with plain
-// delays, 8.43e-8 so and with a delay per pulse; 4096 x 4096 pixels 260 and 265 ms.
+// delays, 8.43e-8 so and with a delay per pulse; 4096 x 4096 pixels 263 and 267 ms.
 struct Delay2 {
     double hi, lo;
 };
@@ -471,14 +471,6 @@ __device__ inline void for_each_tile(const BatchHeader* batch, Body&& body)
 // segment's sum added to the pixel's in order: batches too small to fill the
 // chip give every segment its own wavefront (`seg` >= 0), which leaves its
 // segment's sum in a.parts for plain_total_kernel to add in the same order.
-// How far the cubic may be off the delay (cycles): the phase's own rounding, a
-// few ulp of fc tau, or 6e-9 rad.
-constexpr double kCubicUlps = 8. / 9007199254740992.;
-constexpr double kCubicTol = 1e-9;
-// Largest third difference of the phase (radians) whose phasor 1 + i eps is
-// good to 2e-8 at the chunk's end (eps^2 / 2 times 64^3 / 6).
-constexpr double kCubicEps = 9e-7;
-
 // One lane's pixel of a plain-sum wavefront tile and the pulses [kw0, kw1) the
 // wavefront's pixels integrate.
 struct PlainPixel {
@@ -504,7 +496,7 @@ __device__ inline PlainPixel plain_pixel(const SumArgs& a, const OutDesc& od, in
     return p;
 }
 
-template<int W, bool kExact>
+template<int W, bool kExact, bool kChunks>
 __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const OutDesc& od,
                                   const PlainPixel& px, int seg, int lane)
 {
@@ -588,7 +580,9 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
     // against 64-bit arithmetic is the same.
     // At 850 km, 7.5 km/s and 1520 Hz the cubic is off by 1.4e-10 cycles; a pixel
     // where it is off by more than the tolerance at either of two pulses near its
-    // extrema (short ranges, low PRF) has this chunk's delays evaluated.
+    // extrema has this chunk's delays evaluated.  Where that is to be expected
+    // (short ranges, low PRF) no call tries: 1200 x 1200 pixels at 5 km, 120 m/s and
+    // a PRF of 200 Hz took 16.9 ms with the attempts, 12.9 without.
     // The chunks begin at multiples of kPlainChunk and the choice is the
     // pixel's own, so that its values do not depend on the pixels that share
     // its wavefront.
@@ -598,7 +592,18 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
         tot_im += acc_im;
         acc_re = acc_im = 0.;
     };
-    for (int k = kw0 / kPlainChunk * kPlainChunk; k < kw1; k += kPlainChunk) {
+    // pulse i by its own delay
+    auto single = [&](int i) {
+        const double tau = delay(i);
+        double sn, cs;
+        sincos_turns(a.fc * tau, &sn, &cs);
+        add(i, (tau - a.swst) * a.inv_dtau, cs, sn);
+    };
+    for (int k = kw0; !kChunks && k < kw1; ++k) {
+        if (k % kPlainSeg == 0) end_segment();
+        if (k >= ks && k < ke) single(k);
+    }
+    for (int k = kw0 / kPlainChunk * kPlainChunk; kChunks && k < kw1; k += kPlainChunk) {
         if (k % kPlainSeg == 0) end_segment();
         bool fast = false;
         if ((word(k) & kPosNone) == 0) {
@@ -677,11 +682,7 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
         }
         if (__builtin_amdgcn_ballot_w64(ok && !fast) == 0) continue;
         for (int i = max(k, kw0); i < min(k + kPlainChunk, kw1); ++i) {
-            if (fast || i < ks || i >= ke) continue;
-            const double tau = delay(i);
-            double sn, cs;
-            sincos_turns(a.fc * tau, &sn, &cs);
-            add(i, (tau - a.swst) * a.inv_dtau, cs, sn);
+            if (!fast && i >= ks && i < ke) single(i);
         }
     }
     // found again here, so that it holds no registers in the sum
@@ -707,7 +708,8 @@ __device__ inline void plain_tile(const SumArgs& a, const double2* tab2, const O
 // copied to LDS when it fits kMaxTab2Lds entries.
 constexpr int kMaxTab2Lds = 4096;
 
-template<int W>
+// kChunks false: a delay per pulse throughout (plain_chunks in bp_api.hip).
+template<int W, bool kChunks>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void sum_plain_kernel(SumArgs a)
 {
@@ -733,14 +735,14 @@ void sum_plain_kernel(SumArgs a)
     if (!in_seq) return;
     if (tab_in_lds) {
         if (a.exact_width)
-            plain_tile<W, true>(a, s_tab2, d, px, seg, lane);
+            plain_tile<W, true, kChunks>(a, s_tab2, d, px, seg, lane);
         else
-            plain_tile<W, false>(a, s_tab2, d, px, seg, lane);
+            plain_tile<W, false, kChunks>(a, s_tab2, d, px, seg, lane);
     } else {
         if (a.exact_width)
-            plain_tile<W, true>(a, a.tab2, d, px, seg, lane);
+            plain_tile<W, true, kChunks>(a, a.tab2, d, px, seg, lane);
         else
-            plain_tile<W, false>(a, a.tab2, d, px, seg, lane);
+            plain_tile<W, false, kChunks>(a, a.tab2, d, px, seg, lane);
     }
 }
 
@@ -1605,11 +1607,11 @@ namespace {
 // Kernels of every width kMinKernelWidth..kMaxKernelWidth, indexed by width.
 using Widths = std::make_integer_sequence<int, kMaxKernelWidth - kMinKernelWidth + 1>;
 
-template<int... I>
+template<bool kChunks, int... I>
 const void* plain_fn(int w, std::integer_sequence<int, I...>)
 {
     static const void* const fns[] = {
-        reinterpret_cast<const void*>(&sum_plain_kernel<I + kMinKernelWidth>)...};
+        reinterpret_cast<const void*>(&sum_plain_kernel<I + kMinKernelWidth, kChunks>)...};
     return fns[w - kMinKernelWidth];
 }
 
@@ -1631,7 +1633,7 @@ size_t plain_lds(int ntab) { return ntab <= kMaxTab2Lds ? sizeof(double2) * ntab
 }  // namespace
 
 // Host-side handle of a kernel (0 geometry, 4 geometry for generic DEMs,
-// 1 plain sum, 5 its segments' total, 2 split sum, 3 fit), as graph kernel nodes report it; null for
+// 1 plain sum, 6 with a delay per pulse, 5 its segments' total, 2 split sum, 3 fit), as graph kernel nodes report it; null for
 // a width or variant that is not built.
 const void* kernel_fn(int which, int width, bool staged, bool pair)
 {
@@ -1640,7 +1642,8 @@ const void* kernel_fn(int which, int width, bool staged, bool pair)
     case 4: return reinterpret_cast<const void*>(&geometry_kernel<true>);
     case 5: return reinterpret_cast<const void*>(&plain_total_kernel);
     case 3: return reinterpret_cast<const void*>(&fit_kernel);
-    case 1: return width_ok(width) ? plain_fn(width, Widths{}) : nullptr;
+    case 1: return width_ok(width) ? plain_fn<true>(width, Widths{}) : nullptr;
+    case 6: return width_ok(width) ? plain_fn<false>(width, Widths{}) : nullptr;
     default:
         if (staged) {
             // LDS-staged pulse windows: widths 8 and 9, one line per lane
@@ -1656,7 +1659,7 @@ const void* kernel_fn(int which, int width, bool staged, bool pair)
 hipError_t launch_sum_plain(const SumArgs& args, int width, int grid, int segs, hipStream_t stream)
 {
     if (grid <= 0) return hipSuccess;
-    const void* fn = kernel_fn(1, width, false, false);
+    const void* fn = kernel_fn(args.chunks ? 1 : 6, width, false, false);
     if (fn == nullptr) return hipErrorInvalidValue;
     void* kargs[] = {const_cast<SumArgs*>(&args)};
     hipError_t e = hipLaunchKernel(fn, dim3(grid, std::max(segs, 1)), dim3(256), kargs,

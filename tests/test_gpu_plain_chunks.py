@@ -116,3 +116,43 @@ def test_chunk_phase_against_single_delays(torch_gpu):
     rel = np.linalg.norm(outs[0] - outs[1]) / np.linalg.norm(outs[1])
     print(f"[plain chunks] cubic and single delays differ by {rel:.2e}", flush=True)
     assert rel <= 5.2e-7
+
+
+def test_short_range_low_prf_costs_no_more_than_delays(torch_gpu):
+    """Where no chunk keeps the cubic's tolerance, updates take the time of an
+    evaluated delay each, 1.19 of one by the cubic (measured at 1200 x 1200 pixels;
+    1.48 when every chunk tries its nodes first), alone and in a scene's graph."""
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import KnabKernel, LUT2d, Orbit, TabulatedKernelF32
+    from isce3_amd.focus import Scene, backproject
+    from isce3_amd.geometry import DEMInterpolator
+    t = -50.0 + 10.0 * np.arange(11)
+    pos = np.stack([0 * t + sim.WGS84_A + 3000.0, 0 * t, 120.0 * t], axis=1)
+    orb = Orbit.from_arrays(sim.EPOCH, -50.0, 10.0, pos, np.repeat([[0.0, 0.0, 120.0]], 11, axis=0))
+    na, n = 1000, 1100
+    raw = torch_gpu.ones((na, n + 100), dtype=torch_gpu.complex64, device="cuda:0")
+    out = torch_gpu.empty((n, n), dtype=torch_gpu.complex64, device="cuda:0")
+    kernel, rate = TabulatedKernelF32(KnabKernel(8.0, 0.8), 2048), []
+    for prf in (200.0, 3000.0):
+        ig = RadarGeometry(sim._grid(-0.5 * na / prf, prf, 5000.0, sim.DR, na, n + 100), orb, LUT2d())
+        og = RadarGeometry(sim._grid(-0.5 * n / prf, prf, 5300.0, sim.DR, n, n), orb, LUT2d())
+        best, st = np.inf, {}
+        for _ in range(4):
+            backproject(out, og, raw, ig, DEMInterpolator(50.0), sim.FC, 0.1, kernel, "nodelay",
+                        precision="plain", stats=st)
+            best = min(best, st["sum_ms"] / st["updates"])
+        rate.append(best)
+        part = og.radar_grid.offset_and_resize(100, 200, 33, 65)
+        tile = torch_gpu.empty((33, 65), dtype=torch_gpu.complex64, device="cuda:0")
+        want = torch_gpu.empty_like(tile)
+        backproject(want, RadarGeometry(part, orb, LUT2d()), raw, ig, DEMInterpolator(50.0), sim.FC,
+                    0.1, kernel, "nodelay", precision="plain")
+        with Scene(raw, ig, orb, LUT2d(), DEMInterpolator(50.0), sim.FC, 0.1, kernel, "nodelay",
+                   precision="plain", max_pixels=1 << 12, max_blocks=1) as scene:
+            for _ in range(2):
+                scene.focus([tile], [part])
+                np.testing.assert_array_equal(tile.cpu().numpy(), want.cpu().numpy())
+    print(f"[plain chunks] time per update, single delays over cubic: {rate[0] / rate[1]:.2f}",
+          flush=True)
+    assert rate[0] <= 1.33 * rate[1]
