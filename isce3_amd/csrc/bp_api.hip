@@ -606,6 +606,14 @@ bool fit_line_table(const bp_kernel& k, bp::LineArgs* a)
             for (int q = bp::kEndDegree; q >= 0; --q)
                 r[q] = (q > 0 ? r[q - 1] : 0.) - Fits::E * r[q] + (q == 0 ? ce[d] : 0.);
         }
+        // to the limit of the cell's weights, which imply it for smooth kernels
+        for (int i = 0; i < ME; ++i) {
+            const double past = Fits::E + fits.xe[i];
+            const double want = s == 0 ? weight(hw - past) : value(w0, 0.5 + past);
+            double got = r[bp::kEndDegree];
+            for (int d = bp::kEndDegree - 1; d >= 0; --d) got = got * past + r[d];
+            if (!(std::fabs(got - want) <= 1e-4 * peak)) return false;
+        }
         for (int d = 0; d <= bp::kEndDegree; ++d) (s == 0 ? a->w_in : a->w_out)[d] = (float)r[d];
     }
     return true;
@@ -1169,7 +1177,6 @@ LinePlan plan_lines(const CallArgs& a, int width, const Opts& o)
     const double rmax = 1.02 * (gi.starting_range + gi.width * gi.range_pixel_spacing);
     const double pulses = std::min((double)gi.length, wvl * rmax * ratio / (2. * a.ds) / vmin / dt + 8.);
     p.slots = (int)(pulses / (1 << p.chunk_log2)) + 3;
-    p.table.tropo = a.tropo;
     p.table.n_sums = 8 + (a.tropo != BP_TROPO_NODELAY ? bp::kSlopeNodes : 0);
     p.strip_bytes = bp::line_strip_bytes(p.slots, p.table.n_sums);
     p.on = p.strip_bytes <= kStripBytes;

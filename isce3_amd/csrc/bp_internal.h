@@ -263,7 +263,7 @@ struct LineArgs {
     double2* carry;                      // [strip][segment][64 lines][64]
     int32_t slots;                       // chunks per strip in the workspace
     int32_t chunk_log2;
-    int32_t n_sums, tropo;               // sums per chunk: 8 nodes, and with a
+    int32_t n_sums;                      // sums per chunk: 8 nodes, and with a
                                          // tropospheric delay kSlopeNodes slopes
     float2* sums;                        // [strip][slot][n_sums][64]
     float2* parts;                       // [strip][segment][64 lines][64]

@@ -238,6 +238,46 @@ def test_workspace_bytes(precision, width, max_pixels, least, most):
     assert held(0) <= (9 << 20) + (1 << 20)     # 32 bytes a strip, and one strip
 
 
+def _windowed_sinc(x, width, window):
+    h = width / 2.0
+    w = {"hann": 0.5 + 0.5 * np.cos(np.pi * x / h),
+         "kaiser": np.i0(6.0 * np.sqrt(np.maximum(1 - (x / h) ** 2, 0))) / np.i0(6.0)}[window]
+    return np.sinc(x) * w
+
+
+@pytest.mark.parametrize("width", [8, 9])
+@pytest.mark.parametrize("kind,taken", [
+    (0.3, True), (0.6, True), (0.95, True), ("hann", True), ("kaiser", True),
+    ("box", False), ("steps", False), ("noise", False), ("nan", False), ("triangle", False)])
+def test_kernels_the_line_sum_takes(width, kind, taken):
+    """Knab and windowed-sinc tables of 2048 entries are smooth enough for the
+    weight polynomials (1e-4 of the peak, in the cell and past its ends); tables
+    with steps, kinks in a tap's cell, noise or NaN keep the pixel-by-pixel sum."""
+    from isce3_amd import sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.focus import geometry_struct
+    geometry = RadarGeometry(sim._grid(-2.5, sim.PRF, sim.R0, sim.DR, 8192, 16384),
+                             sim.straight_orbit(), core.LUT2d())
+    n, h = 2048, width / 2.0
+    x = h / (n - 1) * np.arange(n)
+    if isinstance(kind, float):
+        table = core.TabulatedKernelF32(core.KnabKernel(float(width), kind), n).table
+    elif kind in ("hann", "kaiser"):
+        table = _windowed_sinc(x, width, kind)
+    else:
+        table = {"box": np.ones(n), "steps": np.round(np.sinc(x) * 64) / 64,
+                 "triangle": np.maximum(1 - np.abs(x - 0.1), 0),
+                 "noise": np.random.default_rng(1).standard_normal(n),
+                 "nan": np.where(np.arange(n) == 700, np.nan, np.sinc(x))}[kind]
+        table[-1] = 0.0
+    table = np.ascontiguousarray(table, np.float32)
+    kr = _native.Kernel_t(h, n, 0, table.ctypes.data)
+    ig = geometry_struct(geometry)
+    held = _native.lib().bp_workspace_bytes(C.byref(ig), sim.FC, 6.0, C.byref(kr), 1,
+                                            _native.PRECISION_SPLIT, 1 << 20, 64, 1, -1)
+    assert (held > 0) == taken, held
+
+
 @pytest.mark.parametrize("width", [8, 9])
 def test_line_plan_host_time(width):
     """The plan of the line-interpolated sum, which every split call makes
