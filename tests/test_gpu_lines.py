@@ -23,7 +23,8 @@ pytestmark = pytest.mark.gpu
 NA, NR = 4600, 192
 
 
-def _scene(width=8, orbit="straight", relief=0.0, doppler=0.0):
+def _scene(width=8, orbit="straight", relief=0.0, doppler=0.0, na=NA, bandwidth=0.8,
+           dr=None):
     from isce3_amd import sim
     from isce3_amd.container import RadarGeometry
     from isce3_amd.core import KnabKernel, LUT2d, Orbit, TabulatedKernelF32
@@ -38,7 +39,7 @@ def _scene(width=8, orbit="straight", relief=0.0, doppler=0.0):
             sim.EPOCH, -50.0, 10.0,
             np.stack([r * np.cos(a), 0 * a, r * np.sin(a)], axis=1),
             sim.SPEED * np.stack([-np.sin(a), 0 * a, np.cos(a)], axis=1))
-    in_grid = sim._grid(-0.5 * NA / sim.PRF, sim.PRF, sim.R0, sim.DR, NA, NR)
+    in_grid = sim._grid(-0.5 * na / sim.PRF, sim.PRF, sim.R0, dr or sim.DR, na, NR)
     dem = DEMInterpolator(50.0)
     if relief:
         dem = sim._dem_around(orb, in_grid, 256, 30.0, 0.8, relief, 3)
@@ -46,12 +47,13 @@ def _scene(width=8, orbit="straight", relief=0.0, doppler=0.0):
     ys = np.array([-45.0, 45.0])
     lut = LUT2d(xs, ys, np.full((2, 2), doppler)) if doppler else LUT2d()
     rng = np.random.default_rng(5)
-    raw = (rng.standard_normal((NA, NR)) + 1j * rng.standard_normal((NA, NR))).astype(np.complex64)
-    kernel = TabulatedKernelF32(KnabKernel(float(width), 0.8), 2048)
+    raw = (rng.standard_normal((na, NR)) + 1j * rng.standard_normal((na, NR))).astype(np.complex64)
+    kernel = TabulatedKernelF32(KnabKernel(float(width), bandwidth), 2048)
     return orb, RadarGeometry(in_grid, orb, lut), dem, raw, kernel
 
 
-def _run(scene, rows, cols, c0=40, dr=None, prf=None, tropo="nodelay", options=None):
+def _run(scene, rows, cols, c0=40, dr=None, prf=None, tropo="nodelay", options=None, ds=6.0,
+         bandwidth=0.8):
     """(GPU split result, FP64 oracle) of a block of rows x cols pixels."""
     from isce3_amd import sim
     from isce3_amd.container import RadarGeometry
@@ -63,10 +65,10 @@ def _run(scene, rows, cols, c0=40, dr=None, prf=None, tropo="nodelay", options=N
                      dr or sim.DR, rows, cols)
     og = RadarGeometry(grid, orb, LUT2d())
     out = np.empty(grid.shape, np.complex64)
-    err = backproject(out, og, raw, in_geom, dem, sim.FC, 6.0, kernel, tropo, precision="split",
+    err = backproject(out, og, raw, in_geom, dem, sim.FC, ds, kernel, tropo, precision="split",
                       options=options)
-    ref, _, _, rc = oracle.backproject(og, raw, in_geom, dem, sim.FC, 6.0, kernel, tropo, mode=1,
-                                       kernel_bandwidth=0.8)
+    ref, _, _, rc = oracle.backproject(og, raw, in_geom, dem, sim.FC, ds, kernel, tropo, mode=1,
+                                       kernel_bandwidth=bandwidth)
     assert err == (rc == 6)
     rel = complex_rel_error(out, ref)
     print(f"[lines] {rows}x{cols} rel={rel:.2e}", flush=True)
@@ -86,6 +88,21 @@ def test_strip_edges_match_fp64_oracle(torch_gpu, width, rows, cols):
                                                 ("circular", 100.0, "tsx")])
 def test_orbits_and_terrain_match_fp64_oracle(torch_gpu, orbit, relief, tropo):
     assert _run(_scene(8, orbit, relief), 96, 70, tropo=tropo) <= 1e-4
+
+
+@pytest.mark.parametrize("ds,na,dr,c0", [(5.0, NA + 800, None, 40), (3.0, 8200, None, 60),
+                                         (4.0, 6400, 3.0, 40)])
+@pytest.mark.parametrize("rows,cols,tropo", [(16, 40, "nodelay"), (33, 20, "tsx"), (70, 33, "nodelay")])
+def test_finer_resolutions(torch_gpu, ds, na, dr, c0, rows, cols, tropo):
+    """Strips of 32 lines with 64 pulses per chunk (5 m) and with 32 (3 m), and of 16
+    lines (4 m with a range spacing of 3 m), over whole apertures of 4,600, 7,700 and
+    5,700 pulses that stay inside the range line."""
+    assert _run(_scene(8, na=na, dr=dr), rows, cols, c0=c0, ds=ds, dr=dr, tropo=tropo) <= 6e-5
+
+
+@pytest.mark.parametrize("width,bandwidth", [(8, 0.6), (9, 0.9)])
+def test_other_kernels(torch_gpu, width, bandwidth):
+    assert _run(_scene(width, bandwidth=bandwidth), 50, 64, bandwidth=bandwidth) <= 6e-5
 
 
 @pytest.mark.parametrize("kw", [dict(dr=9.0), dict(prf=400.0), dict(c0=-30), dict(c0=150)])
@@ -166,35 +183,72 @@ def test_grids_without_strips(torch_gpu):
     assert taken(grid(640, 640)) >= 640 * 640 * 112 + (24 << 20)
 
 
-def test_whole_and_band_by_band_agree(torch_gpu):
+@pytest.mark.parametrize("width,ds,na,c0,cols", [(9, 6.0, NA, 40, 70), (8, 3.0, 8200, 60, 40),
+                                                 (8, 6.0, NA, -30, 130)])
+def test_whole_and_band_by_band_agree(torch_gpu, width, ds, na, c0, cols):
     """Pulses in host memory under a budget below a strip's window: the strip's
-    pulses go through the device in parts, with the same result to the bit."""
+    pulses go through the device in parts, with the same result to the bit; with
+    chunks of 64 and of 32 pulses, and with strips beside them that are left to the
+    pixel-by-pixel sum (a block that begins before the swath)."""
     from isce3_amd import sim
     from isce3_amd.container import RadarGeometry
     from isce3_amd.core import LUT2d
     from isce3_amd.focus import backproject
-    orb, in_geom, dem, raw, kernel = _scene(9)
-    grid = sim._grid(-0.5 * 150 / sim.PRF, sim.PRF, sim.R0 + 40 * sim.DR, sim.DR, 150, 70)
+    orb, in_geom, dem, raw, kernel = _scene(width, na=na)
+    grid = sim._grid(-0.5 * 150 / sim.PRF, sim.PRF, sim.R0 + c0 * sim.DR, sim.DR, 150, cols)
     og = RadarGeometry(grid, orb, LUT2d())
+    lines = 64 if ds >= 6 else 32
     outs = []
-    # whole; bands of one strip row each (64 lines' window); parts of a strip's window
+    # whole; bands of one strip row each (its lines' window); parts of a strip's window
     windows = [0]
     for windows_of in (0, 1, 2):
         budget = windows[windows_of] * NR * 8
         out = np.empty(grid.shape, np.complex64)
         st = {}
-        backproject(out, og, raw, in_geom, dem, sim.FC, 6.0, kernel, "nodelay",
+        backproject(out, og, raw, in_geom, dem, sim.FC, ds, kernel, "nodelay",
                     precision="split", max_window_bytes=budget, stats=st)
         print(f"[lines] budget {budget}: {st['bands']} bands, {st['window_pulses']} pulses",
               flush=True)
         outs.append(out)
         if not windows_of:
-            strip = st["window_pulses"] - 150 + 64
-            windows += [strip + 20, strip - 40]
+            strip = st["window_pulses"] - 150 + lines
+            windows += [strip + lines // 2, strip - lines // 2]
         else:
             assert st["bands"] >= 2
     np.testing.assert_array_equal(outs[1], outs[0])
     np.testing.assert_array_equal(outs[2], outs[0])
+
+
+def test_groups_of_one_strip_agree(torch_gpu):
+    """A context whose workspace is limited to one strip runs a block of 18 strips
+    in as many groups, with the same result to the bit."""
+    import ctypes as C
+    from isce3_amd import _native, sim
+    from isce3_amd.container import RadarGeometry
+    from isce3_amd.core import LUT2d
+    from isce3_amd.focus import geometry_struct, parse_geo2rdr_params, parse_rdr2geo_params
+    orb, in_geom, dem, raw, kernel = _scene(8)
+    d_raw = torch_gpu.from_numpy(raw).to("cuda:0")
+    geom = RadarGeometry(sim._grid(-0.2, sim.PRF, sim.R0 + 40 * sim.DR, sim.DR, 64 * 6, 130), orb,
+                         LUT2d())
+    og, ig, dm, kr = geometry_struct(geom), geometry_struct(in_geom), dem._struct(), kernel._struct()
+    r2g, g2r = parse_rdr2geo_params({}), parse_geo2rdr_params({})
+    lib, outs = _native.lib(), []
+    for limit in (-1, 0):
+        ctx, failed, opt, st = C.c_void_p(), C.c_int(0), _native.Options_t(), _native.Stats_t()
+        _native.check(lib.bp_context_create(0, C.byref(ctx)))
+        _native.check(lib.bp_context_limit_workspace(ctx, limit))
+        out = torch_gpu.empty((64 * 6, 130), dtype=torch_gpu.complex64, device="cuda:0")
+        torch_gpu.cuda.synchronize()
+        rc = lib.bp_backproject(ctx, C.byref(og), C.byref(ig), C.byref(dm), sim.FC, 6.0, C.byref(kr),
+                                0, C.byref(r2g), C.byref(g2r), C.c_void_p(d_raw.data_ptr()),
+                                C.c_void_p(out.data_ptr()), None, _native.PRECISION_SPLIT,
+                                C.byref(opt), None, C.byref(failed), C.byref(st))
+        lib.bp_context_destroy(ctx)
+        _native.check(rc)
+        outs.append(out.cpu().numpy())
+    np.testing.assert_array_equal(outs[1], outs[0])
+    assert np.isfinite(outs[0]).all()
 
 
 @pytest.mark.parametrize("width,tropo", [(8, "nodelay"), (9, "tsx")])
