@@ -45,6 +45,7 @@ LINE_FLOPS_PER_UPDATE = (256 + 8 * 40) / 64
 PEAK_FP32_TFLOPS = 157.3
 PEAK_FP64_TFLOPS = 78.6
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "sum_split_kernel_two_lines_pmc.md")
+LINE_TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "strip_kernels_pmc.md")
 STAGE_TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "hbm_traffic_rangecomp_rslc_presum.md")
 
 
@@ -52,15 +53,16 @@ def log(msg):
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
 
 
-def hbm_bytes_per_launch():
-    """HBM bytes per launch of the split sum kernel on the headline workload,
-    from the committed rocprofv3 counter summary (FETCH_SIZE and WRITE_SIZE
-    scaled by a copy-kernel calibration); None when it is absent."""
+def hbm_bytes_per_launch(by_lines):
+    """HBM bytes of the split sum on the headline workload (of a step's line
+    sum, or of a launch of the pixel-by-pixel kernel), from the committed
+    rocprofv3 counter summary (FETCH_SIZE and WRITE_SIZE scaled by a copy-kernel
+    calibration); None when it is absent."""
     try:
-        text = open(TRAFFIC_PROFILE).read()
+        text = open(LINE_TRAFFIC_PROFILE if by_lines else TRAFFIC_PROFILE).read()
     except OSError:
         return None
-    m = re.search(r"HBM bytes per launch:\s*([0-9.eE+]+)", text)
+    m = re.search(r"HBM bytes per (?:launch|step):\s*([0-9.eE+]+)", text)
     return float(m.group(1)) if m else None
 
 
@@ -778,7 +780,7 @@ def main():
         "roofline": {"bound": "valu", "kernel": split_kernel_name(sp["options"]),
                      "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP32_TFLOPS,
-                     "flops_per_update": flops, "traffic": None if by_lines else hbm_bytes_per_launch()},
+                     "flops_per_update": flops, "traffic": hbm_bytes_per_launch(by_lines)},
         "latency": latency,
         "batch": batch,
         "serve": serve_res,

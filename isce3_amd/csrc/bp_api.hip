@@ -1193,8 +1193,8 @@ void use_plan(Opts& o, const LinePlan& p)
 
 // Segments of the plain sum that get wavefronts of their own (0: none).  The
 // chip holds 4,096 of its wavefronts: 256 x 256 pixels are 1,024, each with
-// 512 pulses to sum one after the other, and 301 x 1003 pixels are 4,718, so that
-// a second round runs 15% full.  By segments these take 0.34 instead of
+// 512 pulses to sum one after the other, and 301 x 1003 pixels are 4,816, so that
+// a second round runs 18% full.  By segments these take 0.34 instead of
 // 0.50 ms and 5.8 instead of 8.3 ms.  From four rounds on (kPlainWaves) the
 // last one costs less than the segments' sums, which are kept while they fit
 // kPartBytes.

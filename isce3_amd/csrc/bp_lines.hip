@@ -30,17 +30,17 @@
 // pulses per crossed bin on a line y lines off the reference: 8 % of the
 // pulse-line pairs at 850 km, 7.5 km/s and 4,000 pulses.
 //
-// Every pass is bound by VALU issue.  Work per pixel-pulse at those figures, in
-// VALU instruction slots (a transcendental counts 4): nodes 8/64 x (29 + 14
-// for the shared weight polynomials), lines 3/4, corrections 2 to 3, aperture
-// ends 1, against 52 of the sum that evaluates every pixel at every pulse
-// (bp_kernels.hip).  Measured for 4096 x 4096 pixels of 16384 x 16384 pulses
-// (width 8): fit 0.75, nodes 7.6, lines 9.5, ends 2.3, sum 0.17 ms, together
-// 20.3 ms against 88.0 (fit and sum) pixel by pixel, at 1e-5 instead of 1.2e-4
-// relative error on noise; a 32 x 32 tile 0.26 ms against 2.3 for the whole
+// Measured for 4096 x 4096 pixels of 16384 x 16384 pulses (width 8), with VALU
+// instructions per pixel-pulse: fit 0.88 ms (0.1), nodes 7.4 (5.0), lines 9.6
+// (3.3), ends 2.3 (0.9), sum 0.17, together 20.3 ms against 88.0 (45) pixel by
+// pixel, at 1e-5 instead of 1.2e-4 relative error on noise.  The nodes are bound
+// by VALU issue (1.27 instructions per SIMD and four cycles); the lines by what
+// they read, their records for every chunk and the node sums in each of a strip's
+// 16 line groups (36 GB past L2 at 3.8 TB/s; VALU 0.60); the ends and the fit by
+// latency (0.67 and 0.26).  A 32 x 32 tile takes 0.24 ms against 2.3 for the whole
 // call, because its chunks run in parallel where a wavefront walked the whole
 // aperture of its pixels.  64 lines per strip and 64 pulses per chunk: strips
-// of 32 lines cost the nodes 9 slots per pixel-pulse instead of 5.4 and halve
+// of 32 lines cost the nodes 9 instructions per pixel-pulse instead of 5 and halve
 // the corrections (the same sum), chunks of 32 pulses double the lines' part.
 //
 // Pixels whose tropospheric delays differ sit up to 2e-3 bin off the positions

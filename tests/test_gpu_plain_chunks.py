@@ -5,8 +5,8 @@ tracks where the cubic fits all, none or some of the pixels.
 
 Tolerance: weights and products in FP32, up to 9 taps of 6e-8 each in weight, product
 and sum, add as random errors to at most 3e-7 of a pixel; a cubic within 1e-9
-cycles (6e-9 rad) or a few ulp of the phase (1e-8 rad) and a phasor within 2e-8
-are below that: 5e-7."""
+cycles (6e-9 rad) or 8 ulp of the phase (4e-8 rad at 850 km) and a phasor within
+2e-8 are below that: 5e-7."""
 import numpy as np
 import pytest
 
