@@ -2151,9 +2151,12 @@ extern "C" int64_t bp_workspace_bytes(const bp_radar_geometry* ig, double fc, do
 try {
     // the rules of check_call that the plans below rely on
     if (ig == nullptr || kernel == nullptr || !(ig->grid.prf > 0) || !(fc > 0) || !(ds > 0) ||
-        kernel->n < 2 || kernel->table == nullptr || !(kernel->halfwidth > 0) || ig->orbit.n < 2 ||
-        ig->orbit.pos == nullptr || ig->orbit.vel == nullptr || max_pixels < 1 || max_blocks < 1)
+        kernel->n < 2 || kernel->table == nullptr || !(kernel->halfwidth > 0) || max_pixels < 1 ||
+        max_blocks < 1)
         return fail(BP_ERR_INVALID_ARGUMENT, "invalid argument");
+    int rc;
+    if ((rc = check_orbit(ig->orbit, "input geometry")) != BP_SUCCESS) return rc;
+    if ((rc = check_lut(ig->doppler, "input geometry")) != BP_SUCCESS) return rc;
     CallArgs a{nullptr, nullptr, ig, nullptr, fc, ds, kernel, dry_tropo_model, nullptr, nullptr,
                nullptr, precision};
     if (precision == BP_PRECISION_PLAIN) {

@@ -151,8 +151,7 @@ class GpuExecutor:
                 C.byref(ig), float(raw.fc), float(raw.ds), C.byref(kr),
                 parse_dry_tropo_model(raw.dry_tropo_model), _PRECISION[precision],
                 int(max_batch_pixels), int(max_batch_requests), int(self.graphs), int(limit))
-            _native.check(min(n, 0))
-            sizes.append(n)
+            sizes.append(max(n, 0))   # a set that no call accepts fails its requests
         return sum(sizes) if self.graphs else max(sizes, default=0)
 
     def configure(self, max_batch_pixels: int, max_batch_requests: int, workspace: int = -1):

@@ -235,6 +235,9 @@ def test_workspace_bytes(precision, width, max_pixels, least, most):
     assert least <= held(-1) <= most
     assert held(-1) <= held(-1, 0) <= (3 << 29) + (9 << 20)   # a context's calls of any shape
     assert held(10 << 20) <= max(10 << 20, (9 << 20) + (1 << 20))
+    ig.doppler.have_data, ig.doppler.width = 1, 1      # refused as the calls refuse it
+    assert held(-1) == _native.BP_ERR_INVALID_ARGUMENT
+    ig.doppler.have_data = 0
     assert held(0) <= (9 << 20) + (1 << 20)     # 32 bytes a strip, and one strip
 
 
