@@ -467,7 +467,7 @@ class Scene:
     must stay alive and unchanged), ``in_geometry``, the output ``out_orbit``
     and ``out_doppler``, ``dem``, ``fc``, ``ds``, ``kernel``, the troposphere
     model and solver parameters.  Orbits, Doppler tables, DEM and kernel
-    tables are uploaded once; per-pixel scratch is reserved for up to
+    tables are uploaded once; per-pixel scratch and workspace are reserved for up to
     ``max_pixels`` pixels in up to ``max_blocks`` output blocks per call.
     :meth:`focus` gives, block for block, the result of
     :func:`backproject_blocks` with the same arguments.  One host thread at a

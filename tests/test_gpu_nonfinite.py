@@ -81,3 +81,27 @@ def test_host_pulses_in_parts(torch_gpu):
     assert part_st["bands"] > 2
     np.testing.assert_array_equal(got, _focus(sc, raw))
     assert np.isnan(got).any() and np.isfinite(whole).all()
+
+
+def test_scene_replays(torch_gpu):
+    """In a scene's graph and in batches, as in a call of its own."""
+    from isce3_amd import sim
+    from isce3_amd.focus import Scene, backproject_blocks
+    sc = _scene()
+    og, ig, dem, raw, kernel = sc
+    raw = raw.copy()
+    raw[700, 80] = np.inf
+    d_raw = torch_gpu.from_numpy(raw).to("cuda:0")
+    want = _focus(sc, raw)
+    outs = [torch_gpu.empty((ROWS, COLS), dtype=torch_gpu.complex64, device="cuda:0")
+            for _ in range(2)]
+    backproject_blocks(outs, [og, og], d_raw, ig, dem, sim.FC, 6.0, kernel, "nodelay",
+                       precision="split")
+    for o in outs:
+        np.testing.assert_array_equal(o.cpu().numpy(), want)
+    with Scene(d_raw, ig, og.orbit, og.doppler, dem, sim.FC, 6.0, kernel, "nodelay",
+               precision="split", max_pixels=ROWS * COLS, max_blocks=1) as scene:
+        for _ in range(3):
+            outs[0].zero_()
+            scene.focus(outs[:1], [og.radar_grid])
+            np.testing.assert_array_equal(outs[0].cpu().numpy(), want)
